@@ -9,10 +9,10 @@
 // transposed copy of the weights (the reference makes one, ratchet.py:52).
 //
 // Two kernels:
-//  * int8_gemm_m32_kernel, for aligned shapes (K % 64 == 0, 16-byte aligned rows and
+//  * int8_gemm_m32_kernel, for aligned shapes (K % 16 == 0, 16-byte aligned rows and
 //    scales, N % 8 == 0): v_mfma_i32_32x32x32_i8, 128 x 128 or 256 x 256 block tiles, buffer
 //    addressing, register ring + LDS ping-pong, LDS-staged coalesced epilogue;
-//  * int8_gemm_nt_kernel, any shape and stride (ragged K, unaligned rows):
+//  * int8_gemm_nt_kernel, any shape and stride (K % 16 != 0, unaligned rows):
 //    v_mfma_i32_16x16x64_i8 with bounds-checked staging.
 // Block order is XCD-aware: consecutive tile indices (which share an A row panel)
 // are kept on one XCD's L2.
@@ -220,6 +220,9 @@ __global__ __launch_bounds__(256) void int8_gemm_nt_kernel(GemmArgs g) {
   }
 }
 
+// A buffer offset past every descriptor (all are below 2^31 bytes): loads read zeros.
+constexpr int kPastBuffer = static_cast<int>(0x80000000u);
+
 // Staging registers of one k-step (one slot of the register ring).
 template <int NA, int NB>
 struct RingSlot {
@@ -266,7 +269,13 @@ using CfgBig = M32Cfg<256, 256, 2, 4, 2, 2, 1>;
 //    copy-out covers 64 banks, so neither side needs a swizzle or a lane swap;
 //  * each thread copies out a fixed 8-column chunk, so the column bound is one compare.
 // ---------------------------------------------------------------------------
-template <int KIND, int CDT, bool HAS_RS, class CFG>
+//
+// TAIL: K % 64 != 0 (K % 16 == 0). The last k-step's A segments past K are requested at an
+// offset past the descriptor, which reads zeros, so whatever B holds there (the next row's
+// bytes) contributes nothing to the int32 sums. One select per load, instead of the
+// byte-wise general kernel these shapes took before (5003 x 1040 x 2768 packed: 290 us; the
+// NT form of its grad_input, 5003 x 2768 x 1040: 416 us).
+template <int KIND, int CDT, bool HAS_RS, class CFG, bool TAIL>
 __global__ __launch_bounds__(CFG::THREADS) __attribute__((amdgpu_waves_per_eu(CFG::MINW, 8)))
 void int8_gemm_m32_kernel(GemmArgs g) {
   constexpr int BM = CFG::BM, BN = CFG::BN, BK = 64, S = CFG::RING;
@@ -311,6 +320,11 @@ void int8_gemm_m32_kernel(GemmArgs g) {
       BT ? make_buffer(g.B + n0, (g.K - 1) * g.ldb + (g.N - n0))
          : make_buffer(g.B + n0 * g.ldb, (rows_b - 1) * g.ldb + g.K);
   const int b_step = BT ? BK * static_cast<int>(g.ldb) : BK;
+  static_assert(!(BT && TAIL), "the packed [K, N] operand has whole k-steps");
+  const int nk = TAIL ? static_cast<int>((g.K + BK - 1) / BK) : static_cast<int>(g.K / BK);
+  // this thread's A segment (the same for every piece: THREADS % 4 == 0) lies past K in the
+  // last k-step
+  const bool past_k = TAIL && 16 * (tid & 3) >= static_cast<int>(g.K) - (nk - 1) * BK;
   int a_voff[SEGS], b_voff[SEGS], st_off[SEGS], bst_off[SEGS];
 #pragma unroll
   for (int j = 0; j < SEGS; ++j) {
@@ -331,8 +345,9 @@ void int8_gemm_m32_kernel(GemmArgs g) {
   auto load = [&](RingSlot<SEGS, SEGS>& r, int kt) {
 #pragma unroll
     for (int j = 0; j < SEGS; ++j)
-      r.a[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                             a_rsrc, a_voff[j], kt * BK, 0));
+      r.a[j] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     a_rsrc, TAIL && past_k && kt == nk - 1 ? kPastBuffer : a_voff[j], kt * BK, 0));
 #pragma unroll
     for (int j = 0; j < SEGS; ++j)
       r.b[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
@@ -384,7 +399,6 @@ void int8_gemm_m32_kernel(GemmArgs g) {
     const __amdgpu_buffer_rsrc_t rs_rsrc = make_buffer(g.rs + n0, rows_b * 4);
     rsv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_rsrc, tid * 4, 0, 0));
   }
-  const int nk = static_cast<int>(g.K / BK);
   if constexpr (S == 2) {
     load(ring[0], 0);
     __builtin_amdgcn_sched_barrier(0);
@@ -572,7 +586,8 @@ struct PipeSched {
   int tiles, tiles_m, tiles_n, tiles_per_xcd;
 };
 
-template <int KIND, int CDT, bool HAS_RS>
+// TAIL: K % 64 != 0, as in the ring kernel (the last k-step's A segments past K read zeros).
+template <int KIND, int CDT, bool HAS_RS, bool TAIL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void int8_gemm_pipe_kernel(GemmArgs g, PipeSched p) {
   constexpr int BM = kPipeBM, BN = kPipeBN, BK = kPipeBK, S = kPipeStages;
@@ -596,7 +611,8 @@ void int8_gemm_pipe_kernel(GemmArgs g, PipeSched p) {
   const int t_begin = xcd * p.tiles_per_xcd;
   const int t_span = min(p.tiles, t_begin + p.tiles_per_xcd) - t_begin;
   const int n_my = t_span > lb ? (t_span - lb + bpx - 1) / bpx : 0;
-  const int nk = static_cast<int>(g.K / BK);
+  static_assert(!(BT && TAIL), "the packed [K, N] operand has whole k-steps");
+  const int nk = TAIL ? static_cast<int>((g.K + BK - 1) / BK) : static_cast<int>(g.K / BK);
   const int total = n_my * nk;
 
   // Per-lane DMA source offsets (fixed for the kernel). Wave w fills 1 KB chunks 2w and
@@ -616,6 +632,7 @@ void int8_gemm_pipe_kernel(GemmArgs g, PipeSched p) {
     }
   }
   const int b_kstep = BT ? BK * ldb : BK;  // B offset per k-step
+  const bool past_k = TAIL && 16 * sg >= static_cast<int>(g.K) - (nk - 1) * BK;
 
   // Tile order: groups of GM row tiles, n-major inside a group, so the 32 tiles an XCD
   // runs at once span GM row panels of A and 32 / GM column panels of B.
@@ -655,7 +672,8 @@ void int8_gemm_pipe_kernel(GemmArgs g, PipeSched p) {
     const uint32_t st = lds0 + pstage * STAGE + 1024 * CH * wave;
     const int ak = pk * BK, bk = pk * b_kstep;
 #pragma unroll
-    for (int c = 0; c < CH; ++c) dma16(ar, st + 1024 * c, a_v[c] + ak, 0);
+    for (int c = 0; c < CH; ++c)
+      dma16(ar, st + 1024 * c, TAIL && past_k && pk == nk - 1 ? kPastBuffer : a_v[c] + ak, 0);
 #pragma unroll
     for (int c = 0; c < CH; ++c) dma16(br, st + ASZ + 1024 * c, b_v[c] + bk, 0);
     if (++pstage == S) pstage = 0;
@@ -959,7 +977,7 @@ static bool use_pipe(const GemmArgs& g, int es) {
   return g.N >= 4096 && tiles >= 256;
 }
 
-template <int KIND, int CDT, bool HAS_RS>
+template <int KIND, int CDT, bool HAS_RS, bool TAIL>
 static void launch_pipe(const GemmArgs& g, hipStream_t stream) {
   PipeSched p{};
   p.tiles_n = static_cast<int>((g.N + kPipeBN - 1) / kPipeBN);
@@ -968,33 +986,48 @@ static void launch_pipe(const GemmArgs& g, hipStream_t stream) {
   p.tiles_per_xcd = (p.tiles + 7) / 8;
   // one 512-thread block per CU (256 CUs), 8 per XCD at least; never more blocks than tiles
   const int per_xcd = p.tiles_per_xcd < 32 ? p.tiles_per_xcd : 32;
-  int8_gemm_pipe_kernel<KIND, CDT, HAS_RS><<<dim3(8 * per_xcd), 512, 0, stream>>>(g, p);
+  int8_gemm_pipe_kernel<KIND, CDT, HAS_RS, TAIL><<<dim3(8 * per_xcd), 512, 0, stream>>>(g, p);
 }
 
-template <int KIND, int CDT, bool HAS_RS>
-static void launch_m32(const GemmArgs& g, hipStream_t stream) {
+template <int KIND, int CDT, bool HAS_RS, bool TAIL>
+static void launch_tiles(const GemmArgs& g, hipStream_t stream) {
   if (use_pipe(g, CDT == RK_BF16 ? 2 : 4)) {
-    launch_pipe<KIND, CDT, HAS_RS>(g, stream);
+    launch_pipe<KIND, CDT, HAS_RS, TAIL>(g, stream);
     return;
   }
   if (use_big_tiles(g)) {
     const int64_t tiles = ((g.M + 255) / 256) * ((g.N + 255) / 256);
-    int8_gemm_m32_kernel<KIND, CDT, HAS_RS, CfgBig>
+    int8_gemm_m32_kernel<KIND, CDT, HAS_RS, CfgBig, TAIL>
         <<<dim3(static_cast<unsigned>(tiles)), CfgBig::THREADS, 0, stream>>>(g);
   } else {
     const int64_t tiles = ((g.M + 127) / 128) * ((g.N + 127) / 128);
-    int8_gemm_m32_kernel<KIND, CDT, HAS_RS, CfgSmall>
+    int8_gemm_m32_kernel<KIND, CDT, HAS_RS, CfgSmall, TAIL>
         <<<dim3(static_cast<unsigned>(tiles)), CfgSmall::THREADS, 0, stream>>>(g);
   }
 }
 
+template <int KIND, int CDT, bool HAS_RS>
+static void launch_m32(const GemmArgs& g, hipStream_t stream) {
+  if constexpr (KIND != B_PACKED_T) {
+    if (g.K % kBK != 0) {
+      launch_tiles<KIND, CDT, HAS_RS, true>(g, stream);
+      return;
+    }
+  }
+  launch_tiles<KIND, CDT, HAS_RS, false>(g, stream);
+}
+
 template <int KIND, int CDT>
 static int launch_gemm(const GemmArgs& g, hipStream_t stream) {
-  const bool fast = (g.K % kBK) == 0 && (g.lda % 16) == 0 && (g.ldb % 16) == 0 &&
-                    aligned16(g.A) && aligned16(g.B);
+  const bool rows16 = (g.lda % 16) == 0 && (g.ldb % 16) == 0 && aligned16(g.A) && aligned16(g.B);
+  const bool fast = (g.K % kBK) == 0 && rows16;
   const int es = CDT == RK_BF16 ? 2 : 4;
-  const bool aligned_out = fast && (g.N % 8) == 0 && ((g.ldc * es) % 16) == 0 &&
+  // K % 16 == 0 with a ragged last k-step takes the tiled kernels too (TAIL); the residual
+  // epilogue and the small-M kernel keep whole k-steps
+  const bool aligned_k16 = rows16 && (g.K % 16) == 0 && (g.N % 8) == 0 &&
+                           ((g.ldc * es) % 16) == 0 &&
                            aligned16(g.C) && (g.rs == nullptr || aligned16(g.rs));
+  const bool aligned_out = aligned_k16 && fast;
   // Buffer offsets are 32-bit: a block's furthest A/B load (256 rows, prefetch two
   // k-steps past K) and C store (256 rows) must stay below 2^31 bytes.
   const bool fits32 = 256 * g.lda + g.K + 256 < (int64_t{1} << 31) &&
@@ -1019,7 +1052,7 @@ static int launch_gemm(const GemmArgs& g, hipStream_t stream) {
     else launch_gemv<KIND, CDT, false>(g, stream);
     return launch_status("int8_gemv");
   }
-  if (aligned_out && fits32) {
+  if (fits32 && (aligned_out || (aligned_k16 && g.M > 16))) {
     const int64_t tiles = ((g.M + 127) / 128) * ((g.N + 127) / 128);
     if (tiles > 0x7fffffff) return fail(RK_ERR_ARG, "GEMM grid too large");
     if (g.rs) launch_m32<KIND, CDT, true>(g, stream);
