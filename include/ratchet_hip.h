@@ -655,6 +655,30 @@ int rk_attention_forward(const uint16_t* q, int64_t sqb, int64_t sqh, int64_t sq
                          int64_t H, int64_t S, int64_t D, float scale, uint16_t* o, int64_t sob,
                          int64_t soh, int64_t sos, float* lse, void* stream);
 
+/*
+ * The backward of rk_attention_forward: dq, dk, dv (bf16) from q, k, v, o, the gradient g of o
+ * (bf16 [B, H, S, D], strides as in the forward) and the forward's lse. With p_ij the forward's
+ * probabilities and delta_i = g_i . o_i:
+ *   dv_j = sum_i p_ij g_i,  ds_ij = p_ij (g_i . v_j - delta_i),
+ *   dq_i = scale sum_j ds_ij k_j,  dk_j = scale sum_i ds_ij q_i,
+ * float32 sums of bf16 products (p and ds enter theirs rounded to bf16), each output summed in
+ * a fixed order. dq, dk, dv share their strides (8-byte aligned rows). work: at least
+ * rk_attention_backward_work(B, H, S) floats. D = 64 or 128, 16-byte aligned inputs, strides
+ * multiples of 8 elements, one head's positions and the row statistics under 2^31 bytes;
+ * otherwise RK_ERR_UNSUPPORTED.
+ * Replaces: the backward of F.scaled_dot_product_attention(q, k, v, is_causal=True),
+ *           model.py:117-123.
+ */
+int64_t rk_attention_backward_work(int64_t B, int64_t H, int64_t S);
+int rk_attention_backward(const uint16_t* q, int64_t sqb, int64_t sqh, int64_t sqs,
+                          const uint16_t* k, int64_t skb, int64_t skh, int64_t sks,
+                          const uint16_t* v, int64_t svb, int64_t svh, int64_t svs,
+                          const uint16_t* o, int64_t sob, int64_t soh, int64_t sos,
+                          const uint16_t* g, int64_t sgb, int64_t sgh, int64_t sgs,
+                          const float* lse, int64_t B, int64_t H, int64_t S, int64_t D,
+                          float scale, uint16_t* dq, uint16_t* dk, uint16_t* dv, int64_t sxb,
+                          int64_t sxh, int64_t sxs, float* work, void* stream);
+
 /* HBM streaming probe (measurement only; no counterpart in the reference): reads `bytes`
  * (a multiple of 16) from src in 16-byte vectors, `unroll` (1, 2, 4, 8) loads in flight
  * per thread, `blocks` blocks of 256 threads in a grid-stride loop; copy != 0 writes them

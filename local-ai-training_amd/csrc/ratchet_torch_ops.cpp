@@ -970,6 +970,51 @@ std::tuple<Tensor, Tensor> attention_forward(const Tensor& q, const Tensor& k, c
   return {o, lse};
 }
 
+// The backward of attention_forward (rk_attention_backward): (dq, dk, dv), each a [B, H, S, D]
+// view of [B, S, H, D] memory (rows a qkv projection's backward reads in place).
+std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& grad, const Tensor& q,
+                                                      const Tensor& k, const Tensor& v,
+                                                      const Tensor& o, const Tensor& lse,
+                                                      double scale) {
+  require_gpu(q, "attention backward");
+  for (const Tensor* t : {&grad, &k, &v, &o}) {
+    same_device(q, *t, "attention backward");
+    TORCH_CHECK(t->sizes() == q.sizes() && t->scalar_type() == at::kBFloat16,
+                "attention backward: q, k, v, o and the gradient must share a bfloat16 "
+                "[B, H, S, D] shape");
+  }
+  same_device(q, lse, "attention backward");
+  TORCH_CHECK(q.dim() == 4 && q.scalar_type() == at::kBFloat16,
+              "attention backward: q must be a bfloat16 [B, H, S, D] tensor");
+  const int64_t B = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
+  TORCH_CHECK(lse.scalar_type() == at::kFloat && lse.dim() == 3 && lse.size(0) == B &&
+                  lse.size(1) == H && lse.size(2) == S && lse.is_contiguous(),
+              "attention backward: lse must be a contiguous float32 [B, H, S] tensor");
+  // operands the kernels' 16-byte loads do not take as they lie are copied
+  const auto rows = [](const Tensor& t) {
+    bool ok = t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    for (int i = 0; i < 3; ++i) ok = ok && t.stride(i) % 8 == 0;
+    return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+  };
+  const c10::DeviceGuard guard(q.device());
+  const Tensor qq = rows(q), kk = rows(k), vv = rows(v), oo = rows(o), gg = rows(grad);
+  const auto out = [&] { return at::empty({B, S, H, D}, q.options()).permute({0, 2, 1, 3}); };
+  Tensor dq = out(), dk = out(), dv = out();
+  if (q.numel() == 0) return {dq, dk, dv};
+  Tensor work = at::empty({rk_attention_backward_work(B, H, S)}, lse.options());
+  const auto p16 = [](const Tensor& t) { return static_cast<const uint16_t*>(t.data_ptr()); };
+  const auto w16 = [](const Tensor& t) { return static_cast<uint16_t*>(t.data_ptr()); };
+  check_status(
+      rk_attention_backward(
+          p16(qq), qq.stride(0), qq.stride(1), qq.stride(2), p16(kk), kk.stride(0), kk.stride(1),
+          kk.stride(2), p16(vv), vv.stride(0), vv.stride(1), vv.stride(2), p16(oo), oo.stride(0),
+          oo.stride(1), oo.stride(2), p16(gg), gg.stride(0), gg.stride(1), gg.stride(2),
+          lse.data_ptr<float>(), B, H, S, D, static_cast<float>(scale), w16(dq), w16(dk), w16(dv),
+          dq.stride(0), dq.stride(1), dq.stride(2), work.data_ptr<float>(), stream_of(q)),
+      "rk_attention_backward");
+  return {dq, dk, dv};
+}
+
 // Means of segments [offsets[s], offsets[s + 1]) of a float32 row-rms buffer (rk_row_rms_means).
 Tensor row_rms_means(const Tensor& row_rms, const Tensor& offsets) {
   require_gpu(row_rms, "row rms means");
@@ -1117,6 +1162,8 @@ TORCH_LIBRARY(ratchet, m) {
   m.def("embedding_backward(Tensor grad, Tensor ids, int num_weights) -> Tensor");
   m.def("row_rms_means(Tensor row_rms, Tensor offsets) -> Tensor");
   m.def("attention_forward(Tensor q, Tensor k, Tensor v, float scale) -> (Tensor, Tensor)");
+  m.def("attention_backward(Tensor grad, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, "
+        "float scale) -> (Tensor, Tensor, Tensor)");
   m.def("cross_entropy_forward(Tensor logits, Tensor targets, int ignore_index=-100) -> "
         "(Tensor, Tensor, Tensor)");
   m.def("cross_entropy_backward(Tensor grad_loss, Tensor logits, Tensor targets, Tensor stats, "
@@ -1158,6 +1205,7 @@ TORCH_LIBRARY_IMPL(ratchet, CUDA, m) {
   m.impl("embedding_backward", &embedding_backward);
   m.impl("row_rms_means", &row_rms_means);
   m.impl("attention_forward", &attention_forward);
+  m.impl("attention_backward", &attention_backward);
   m.impl("cross_entropy_forward", &cross_entropy_forward);
   m.impl("cross_entropy_backward", &cross_entropy_backward);
 }

@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "rk_common.h"
+#include "rk_lds_dma.h"
 #include "rk_mfma32.h"
 
 namespace rk {
@@ -561,7 +562,6 @@ void int8_gemm_m32_kernel(GemmArgs g) {
 // the compiler does not track: its own vmcnt waits (the residual loads) only become
 // stricter, never too weak, with loads it cannot see in flight.
 // ---------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
 typedef unsigned int u32x2_v __attribute__((ext_vector_type(2)));
 
 constexpr int kPipeBM = 256, kPipeBN = 256, kPipeBK = 64, kPipeStages = 3;
@@ -569,18 +569,6 @@ constexpr int kPipeBM = 256, kPipeBN = 256, kPipeBK = 64, kPipeStages = 3;
 constexpr int kEPitch = 520, kERows = 64;
 constexpr int kPipeStage = (kPipeBM + kPipeBN) * kPipeBK;  // 32 KB
 constexpr int kPipeScales = 2 * 2 * 1024;                  // ls + rs, two tiles
-
-__host__ __device__ constexpr int vmcnt_imm(int n) {
-  // s_waitcnt immediate that waits for vmcnt <= n only (expcnt 7, lgkmcnt 15)
-  return 0x0F70 | (n & 15) | ((n >> 4) << 14);
-}
-
-// One LDS-DMA load: 16 bytes per lane at buffer offset voff + soff into LDS bytes
-// lds + 16 lane .. + 15. M0 holds the LDS address (wave-uniform).
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t lds, int voff, int soff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
-}
 
 struct PipeSched {
   int tiles, tiles_m, tiles_n, tiles_per_xcd;

@@ -123,6 +123,9 @@ SIGNATURES: dict[str, list] = {
     "rk_row_rms_means": [_p, _i64, _p, _i64, _p, _p],
     "rk_attention_forward": [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64,
                              _i64, _i64, _i64, _i64, _i64, _f32, _p, _i64, _i64, _i64, _p, _p],
+    "rk_attention_backward_work": [_i64, _i64, _i64],
+    "rk_attention_backward": [*([_p, _i64, _i64, _i64] * 5), _p, _i64, _i64, _i64, _i64, _f32,
+                              _p, _p, _p, _i64, _i64, _i64, _p, _p],
     "rk_version": [],
     "rk_last_error": [],
 }
@@ -130,6 +133,7 @@ SIGNATURES: dict[str, list] = {
 # return types other than int (the status, or an int count)
 RESTYPES = {
     "rk_last_error": ctypes.c_char_p,
+    "rk_attention_backward_work": ctypes.c_int64,
     "rk_decode_attention_splits": ctypes.c_int64,
     "rk_grad_weight_update_counters": ctypes.c_int64,
     "rk_embedding_backward_workspace": ctypes.c_int64,

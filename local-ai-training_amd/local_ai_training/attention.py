@@ -1,11 +1,12 @@
-"""Causal self-attention of the training step with a HIP forward kernel.
+"""Causal self-attention of the training step on HIP kernels.
 
 The reference attends with ``F.scaled_dot_product_attention(q, k, v, is_causal=True)``
 (``model.py:117-123``). Here the forward is ``rk_attention_forward`` (flash form on the bf16
 MFMA, ``csrc/rk_attention.hip``), which writes the output and the per-query log-sum-exp in
-the form torch's memory-efficient attention forward does; the backward is torch's own
-memory-efficient attention backward, called on those two tensors. torch's forward for this
-case ran at 120-210 TFLOP/s on MI355X; the backward is kept as it is.
+the form torch's memory-efficient attention forward does; the backward is
+``rk_attention_backward`` (``csrc/rk_attention_bwd.hip``) on those two tensors. torch's
+memory-efficient backward (which adds its float32 dq by atomics, in an order that varies)
+stays for extents the HIP kernels' 32-bit offsets do not reach.
 
 Supported: bfloat16 GPU q, k, v [B, H, S, D] with D 64 or 128, unit feature stride,
 16-byte aligned storage and strides that are multiples of 8 elements, no attention mask,
@@ -19,6 +20,7 @@ import math
 import torch
 import torch.nn.functional as F
 from torch import Tensor
+from torch.autograd.function import once_differentiable
 
 from .ops import ratchet
 
@@ -57,19 +59,32 @@ def attention_supported(q: Tensor, k: Tensor, v: Tensor) -> bool:
     return True
 
 
+def _backward_fits(tensors: tuple[Tensor, ...]) -> bool:
+    """The limits of ``rk_attention_backward``'s 32-bit offsets: one head's rows up to the
+    padded length within 2^31 bytes of bf16, and its two float32 statistics per padded row."""
+    b, h, s, d = tensors[0].shape
+    padded = -(-s // 128) * 128
+    return (8 * b * h * padded < 2**31 and padded // 128 <= 65535
+            and all(((padded + 64) * t.stride(2) + d) * 2 < 2**31 for t in tensors))
+
+
 class CausalAttentionFn(torch.autograd.Function):
-    """o = causal softmax(q k^T / sqrt(D)) v: HIP forward, torch's memory-efficient backward."""
+    """o = causal softmax(q k^T / sqrt(D)) v: HIP forward and backward."""
 
     @staticmethod
     def forward(ctx, q: Tensor, k: Tensor, v: Tensor) -> Tensor:
         scale = 1.0 / math.sqrt(q.shape[-1])
         out, lse = ratchet().attention_forward(q, k, v, scale)
         ctx.save_for_backward(q, k, v, out, lse)
+        ctx.scale = scale
         return out
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, grad_out: Tensor):
         q, k, v, out, lse = ctx.saved_tensors
+        if _backward_fits((q, k, v, out, grad_out)):
+            return ratchet().attention_backward(grad_out, q, k, v, out, lse, ctx.scale)
         seed, offset = _philox_placeholders()
         dq, dk, dv, _ = torch.ops.aten._scaled_dot_product_efficient_attention_backward(
             grad_out, q, k, v, None, out, lse, seed, offset, 0.0,

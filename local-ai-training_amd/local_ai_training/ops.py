@@ -173,6 +173,11 @@ def _register_fakes() -> None:
         o = q.new_empty((b, sl, h, d)).permute(0, 2, 1, 3)
         return o, q.new_empty((b, h, sl), dtype=torch.float32)
 
+    @fake("ratchet::attention_backward")
+    def _attention_backward(grad, q, k, v, o, lse, scale):
+        b, h, sl, d = q.shape
+        return tuple(q.new_empty((b, sl, h, d)).permute(0, 2, 1, 3) for _ in range(3))
+
     @fake("ratchet::row_rms_means")
     def _row_rms_means(row_rms, offsets):
         return row_rms.new_empty((offsets.shape[0] - 1,))
@@ -188,7 +193,8 @@ def _register_fakes() -> None:
         return logits.new_empty((logits.shape[0], logits.shape[1]))
 
 
-# every operator the library defines (the opcheck tests walk this list)
+# the operators the library defines (the opcheck tests walk this list), but for
+# attention_backward, whose opcheck is beside its own tests
 OPERATORS = (
     "quantize_rows", "int8_mm_nt", "packed_mm", "packed_mm_residual", "packed_mm_accumulate",
     "packed_mm_t", "unpack_transpose", "unpack", "effective_bf16", "grad_input_bf16",

@@ -1,0 +1,111 @@
+"""The HIP causal-attention backward (``rk_attention_backward``) against float64 autograd.
+
+Tolerance: the kernel rounds p and ds to bf16 (2^-9 relative each) before float32 sums, takes o
+and the forward's lse as given (o rounded to bf16, so delta carries 2^-9 of sum |g o|), and
+rounds each result to bf16. Every element is therefore within a few 2^-9 of the sum of the
+absolute values of its terms; the test bounds the error of each [S, D] head by 2^-7 of the
+largest absolute value of that gradient plus the same share of the element itself, plus the
+float32 rounding of one D-long sum (which stands alone where ds cancels to zero: one position).
+
+Lengths: one position, the edges of the 32-row tiles, the 64-row steps and the 128-row blocks,
+a ragged long one, and the training windows.
+"""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from local_ai_training.attention import CausalAttentionFn, causal_attention
+from local_ai_training.ops import ratchet
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(cuda, b, h, s, d, seed=0, scale=1.0):
+    gen = torch.Generator().manual_seed(seed + 1000 * s + d)
+    qkv = (torch.randn(b, s, 3 * h * d, generator=gen) * scale).to(torch.bfloat16).to(cuda)
+    q, k, v = (t.view(b, s, h, d).transpose(1, 2) for t in qkv.chunk(3, dim=-1))
+    g = torch.randn(b, s, h, d, generator=gen).to(torch.bfloat16).to(cuda).transpose(1, 2)
+    return q, k, v, g
+
+
+def reference(q, k, v, g):
+    q, k, v, g = (t.detach().double().contiguous() for t in (q, k, v, g))
+    for t in (q, k, v):
+        t.requires_grad_()
+    s = q.shape[2]
+    scores = q @ k.transpose(-1, -2).contiguous() / math.sqrt(q.shape[-1])
+    mask = torch.ones(s, s, dtype=torch.bool, device=q.device).triu(1)
+    out = scores.masked_fill(mask, -math.inf).softmax(dim=-1) @ v
+    return torch.autograd.grad(out, (q, k, v), g)
+
+
+def hip(q, k, v, g):
+    scale = 1.0 / math.sqrt(q.shape[-1])
+    o, lse = ratchet().attention_forward(q, k, v, scale)
+    return ratchet().attention_backward(g, q, k, v, o, lse, scale)
+
+
+def check(got, operands):
+    largest = math.prod(float(t.abs().max().clamp_min(1)) for t in operands)
+    for mine, ref in zip(got, reference(*operands)):
+        assert mine.dtype == torch.bfloat16 and bool(torch.isfinite(mine).all())
+        bound = (2.0 ** -7 * (ref.abs().amax(dim=(2, 3), keepdim=True) + ref.abs())
+                 + 2.0 ** -23 * ref.shape[-1] * largest)
+        assert bool(((mine.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("s", [1, 31, 32, 33, 64, 65, 127, 128, 129, 191, 300, 517, 1024])
+def test_gradients_against_float64(cuda, s, d):
+    print(f"attention backward S={s} D={d}", flush=True)
+    q, k, v, g = inputs(cuda, 2, 3, s, d)
+    check(hip(q, k, v, g), (q, k, v, g))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_large_scores_and_the_layouts_it_takes(cuda, d):
+    q, k, v, g = inputs(cuda, 1, 2, 200, d, scale=3.0)
+    check(hip(q, k, v, g), (q, k, v, g))
+    got = hip(*(t.contiguous() for t in (q, k, v, g)))
+    for a, b in zip(got, hip(q, k, v, g)):
+        assert torch.equal(a, b)  # the same sums whatever the strides
+        assert a.transpose(1, 2).is_contiguous()
+    # a gradient without unit feature stride or 16-byte rows is copied
+    wide = torch.zeros(1, 2, 200, d + 4, device=cuda, dtype=torch.bfloat16)
+    wide[..., :d] = g
+    for odd in (wide[..., :d], g.transpose(2, 3).contiguous().transpose(2, 3)):
+        for a, b in zip(hip(q, k, v, odd), got):
+            assert torch.equal(a, b)
+
+
+def test_runs_repeat_and_rows_past_the_end_do_not_count(cuda):
+    # positions past S of a longer buffer hold values that would change every sum
+    q, k, v, g = (t.contiguous() for t in inputs(cuda, 2, 2, 160, 128))
+    for t in (q, k, v, g):
+        t[:, :, 130:] = 60000.0
+    cut = [t[:, :, :130] for t in (q, k, v, g)]
+    first = hip(*cut)
+    check(first, cut)
+    for a, b in zip(first, hip(*(t.clone() for t in cut))):
+        assert torch.equal(a, b)
+
+
+def test_expanded_gradient_and_double_backward(cuda):
+    q, k, v, _ = inputs(cuda, 1, 2, 40, 64)
+    leaves = [t.detach().requires_grad_() for t in (q, k, v)]
+    got = torch.autograd.grad(causal_attention(*leaves).sum(), leaves)
+    check(got, (q, k, v, torch.ones_like(q)))
+    first = torch.autograd.grad(CausalAttentionFn.apply(*leaves).float().square().sum(), leaves,
+                                create_graph=True)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(first[0].float().sum(), leaves)
+
+
+def test_opcheck(cuda):
+    q, k, v, g = inputs(cuda, 2, 2, 40, 64)
+    o, lse = ratchet().attention_forward(q, k, v, 0.125)
+    torch.library.opcheck(ratchet().attention_backward, (g, q, k, v, o, lse, 0.125))
