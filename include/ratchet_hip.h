@@ -663,7 +663,7 @@ int rk_attention_forward(const uint16_t* q, int64_t sqb, int64_t sqh, int64_t sq
  *   dq_i = scale sum_j ds_ij k_j,  dk_j = scale sum_i ds_ij q_i,
  * float32 sums of bf16 products (p and ds enter theirs rounded to bf16), each output summed in
  * a fixed order. dq, dk, dv share their strides (8-byte aligned rows). work: at least
- * rk_attention_backward_work(B, H, S) floats. D = 64 or 128, 16-byte aligned inputs, strides
+ * rk_attention_backward_work(B, H, S) floats. D = 128, 16-byte aligned inputs, strides
  * multiples of 8 elements, one head's positions and the row statistics under 2^31 bytes;
  * otherwise RK_ERR_UNSUPPORTED.
  * Replaces: the backward of F.scaled_dot_product_attention(q, k, v, is_causal=True),

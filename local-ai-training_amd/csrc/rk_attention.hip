@@ -2,32 +2,33 @@
 // F.scaled_dot_product_attention(q, k, v, is_causal=True) (model.py:117-123): bf16 q, k, v
 // [B, H, S, D] (any batch / head / position strides, unit feature stride), D = 64 or 128.
 // Writes o (bf16) and the per-query log-sum-exp lse = log(sum_j exp(s_j)) of the scaled
-// scores s_j = (q . k_j) * scale, float32 [B, H, S], the pair torch's memory-efficient
-// attention backward takes (so the backward stays torch's).
+// scores s_j = (q . k_j) * scale, float32 [B, H, S], the pair the backward takes
+// (rk_attention_bwd.hip; torch's memory-efficient attention backward takes the same).
 //
-// One workgroup = 4 wavefronts = 128 queries of one (batch, head); key blocks (64 keys for
-// D = 64, 32 for D = 128) are staged in LDS (K row-major, V transposed). Each wavefront owns 32 queries and computes
-// S^T = K . Q^T with v_mfma_f32_32x32x16_bf16, K rows as the first operand and its Q rows
-// (held in registers) as the second, so a lane holds all the scores of ONE query (its
+// One workgroup = 4 wavefronts = 128 queries of one (batch, head); steps of 64 keys are staged
+// in LDS by DMA, K and V both row-major (rk_attention.h). Each wavefront owns 32 queries and
+// computes S^T = K . Q^T with v_mfma_f32_32x32x16_bf16, K rows as the first operand and its Q
+// rows (held in registers) as the second, so a lane holds all the scores of ONE query (its
 // lane index mod 32) for 16 keys of each 32-key tile (the partner lane l ^ 32 holds the
 // other 16): the softmax's row max and row sum are a lane's own values plus one xor-32
 // exchange. The online softmax runs in base 2 (scores times scale * log2 e, exp2). The
 // output accumulates transposed, O^T = V^T . P^T: the 8 probabilities a lane holds for
 // one 16-key MFMA step are exactly the second operand that step needs, once the
 // operand's k slots are mapped to keys {16 s + 4 h + 0..3, 16 s + 8 + 4 h + 0..3}
-// (h = lane / 32, the accumulator's own row order), and the first operand reads V^T with
-// the same slot order. The probabilities enter the product rounded to bf16; their sum
-// stays float32. Causal blocks above a wavefront's diagonal are skipped; the diagonal
-// block is masked per element. Every global load goes through a buffer descriptor bounded
-// by the (batch, head) extent, so positions past S read zeros without a test.
-#include "rk_common.h"
+// (h = lane / 32, the accumulator's own row order), and the first operand reads V transposed
+// (ds_read_b64_tr_b16) with the same slot order. The probabilities enter the product rounded
+// to bf16; their sum stays float32. Causal tiles above a wavefront's diagonal are skipped; the
+// diagonal step is masked per element. Every global load goes through a buffer descriptor
+// bounded by the (batch, head) extent, so positions past S read zeros without a test.
+//
+// Staging V transposed through registers (16 VALU permutes and 8-byte LDS writes per piece) and
+// its conflicts held the kernel at 36.7 us (B 32, H 8, S 512, D 64) and 112 us (B 8, H 16,
+// S 1024, D 128); both tiles by DMA and V read transposed take 21.2 and 54 us. What is left is
+// about the wavefront's exponentials (7 issue slots per score, as much as its MFMAs at D 128,
+// twice them at D 64) and the operands it reads (26 us for 134 MB at 5.2 TB/s).
+#include "rk_attention.h"
 
 namespace rk {
-
-typedef float v16f_a __attribute__((ext_vector_type(16)));
-typedef __bf16 v8bf_a __attribute__((ext_vector_type(8)));
-
-constexpr int kAttnBM = 128;  // queries per workgroup (4 wavefronts x 32)
 
 struct AttnArgs {
   const uint16_t* q;
@@ -43,213 +44,121 @@ struct AttnArgs {
   float scale_log2;  // scale * log2(e)
 };
 
-__device__ __forceinline__ v8bf_a as_v8bf(uint4 r) { return __builtin_bit_cast(v8bf_a, r); }
-
-typedef __bf16 bf16x2_a __attribute__((ext_vector_type(2)));
-
-// Two finite floats -> a bf16 pair (low half first), round to nearest even: gfx950's
-// packed conversion, one instruction per pair.
-__device__ __forceinline__ uint32_t bf16x2_of(float lo, float hi) {
-  const bf16x2_a v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-  return __builtin_bit_cast(uint32_t, v);
+// op over a lane and its partner lane ^ 32 (the two halves of a query's keys).
+__device__ __forceinline__ float half_max(float v) {
+  const uint32_t b = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float half_sum(float v) {
+  const uint32_t b = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// BN keys per block: 64 for D = 64; 32 for D = 128, which keeps the scores, probabilities
-// and staging registers small enough for two wavefronts per SIMD.
-template <int D, int BN>
-__global__ __launch_bounds__(256) void attn_fwd_kernel(AttnArgs a) {
-  constexpr int BM = kAttnBM, KT = BN / 32;
-  constexpr int KP = D * 2 + 16;  // K row pitch (bytes): 16 rows of a fragment read cover all banks
-  constexpr int VP = BN * 2 + 8;  // V^T row pitch (bytes): the 32 rows of a fragment read are
-                                  // 34 dwords apart, 32 distinct even banks
-  constexpr int PIECES = BN * D / 8 / 256;  // 16-byte pieces of K per thread
-  constexpr int VKEYS = 4, DG = D / 4;       // V staging: 4 keys x 4 features per thread
-  static_assert((BN / VKEYS) * DG == 256, "one 4 x 4 V piece per thread");
-  // two buffers: block kb + 1 is written while block kb is read
-  __shared__ __attribute__((aligned(16))) uint8_t sk2[2][BN * KP];
-  __shared__ __attribute__((aligned(16))) uint8_t sv2[2][D * VP];
-
-  // positions fit 32 bits (checked by the host, with the row offsets of S + BN rows)
+// R keys per step: 64. At D = 128, 32 keys per step took 59 us against 54.
+template <int D, int R>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4)))
+void attn_fwd_kernel(AttnArgs a) {
+  using T = AttnTile<D, R>;
+  constexpr int KT = R / 32;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kAttnStages * 2 * T::BYTES];
+  const uint32_t lds0 = lds_address(smem);
+  // positions fit 32 bits (checked by the host, with the row offsets of S + 128 rows)
   const int S = static_cast<int>(a.S);
-  const int sqs = static_cast<int>(a.sqs), sks = static_cast<int>(a.sks),
-            svs = static_cast<int>(a.svs);
-  const int nqb = (S + BM - 1) / BM;
-  const int qb = nqb - 1 - static_cast<int>(blockIdx.x);  // longest causal rows first
-  const int64_t bh = blockIdx.y;
-  const int64_t b = bh / a.H, h = bh - b * a.H;
-  const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5, l32 = lane & 31;
+  const int64_t BH = a.B * a.H;
+  const int nqb = (S + kAttnRows - 1) / kAttnRows;
+  const int blk = static_cast<int>(blockIdx.x / BH);  // heads fastest: one head stays on an XCD
+  const int qb = nqb - 1 - blk;                       // longest causal rows first
+  const int64_t bh = blockIdx.x - blk * BH, b = bh / a.H, hd = bh - b * a.H;
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q0 = qb * BM;
-  const int qw0 = q0 + 32 * wave;  // this wavefront's first query
-  const int qi = qw0 + l32;        // this lane's query
+  const int qw0 = qb * kAttnRows + 32 * wave, qi = qw0 + l32;  // this lane's query
 
-  // descriptors end at the head's last position: rows past S read zeros (their offsets,
-  // up to S + BN rows, stay below 2^31)
-  const __amdgpu_buffer_rsrc_t qbuf =
-      make_buffer(a.q + b * a.sqb + h * a.sqh, (static_cast<int64_t>(S - 1) * sqs + D) * 2);
-  const __amdgpu_buffer_rsrc_t kbuf =
-      make_buffer(a.k + b * a.skb + h * a.skh, (static_cast<int64_t>(S - 1) * sks + D) * 2);
-  const __amdgpu_buffer_rsrc_t vbuf =
-      make_buffer(a.v + b * a.svb + h * a.svh, (static_cast<int64_t>(S - 1) * svs + D) * 2);
-
-  // Q of this lane's query, features 16 s + 8 hh .. + 7: the second MFMA operand
   v8bf_a qf[D / 16];
-#pragma unroll
-  for (int s = 0; s < D / 16; ++s)
-    qf[s] = as_v8bf(__builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                  qbuf, (qi * sqs + 16 * s + 8 * hh) * 2, 0, 0)));
-
-  // staging. K: piece c = tid + 256 i is row c / (D / 8), features 8 (c % (D / 8)) .. + 7.
-  // V: thread tid takes keys 4 (tid / DG) .. + 3, features 4 (tid % DG) .. + 3 (8-byte loads),
-  // and writes them transposed as 4 rows of V^T, 4 keys (8 bytes) each.
-  uint4 kr[PIECES];
-  uint2 vr[VKEYS];
-  const int vd0 = 4 * (tid % DG), vk0 = VKEYS * (tid / DG);
-  auto gload = [&](int kb) {
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      const int c = tid + 256 * i, row = c / (D / 8), col = 8 * (c % (D / 8));
-      kr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                            kbuf, ((kb * BN + row) * sks + col) * 2, 0, 0));
-    }
-#pragma unroll
-    for (int i = 0; i < VKEYS; ++i)
-      vr[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(
-                                            vbuf, ((kb * BN + vk0 + i) * svs + vd0) * 2, 0, 0));
-  };
-  auto lstore = [&](int buf) {
-    uint8_t* sk = sk2[buf];
-    uint8_t* sv = sv2[buf];
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      const int c = tid + 256 * i, row = c / (D / 8), col = 8 * (c % (D / 8));
-      *reinterpret_cast<uint4*>(sk + row * KP + col * 2) = kr[i];
-    }
-    // feature j of keys vk0 .. vk0 + 3: the low / high halves of word j / 2 of each key
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;  // high or low bf16 halves
-      const uint32_t w0 = (j < 2) ? vr[0].x : vr[0].y, w1 = (j < 2) ? vr[1].x : vr[1].y;
-      const uint32_t w2 = (j < 2) ? vr[2].x : vr[2].y, w3 = (j < 2) ? vr[3].x : vr[3].y;
-      *reinterpret_cast<uint2*>(sv + (vd0 + j) * VP + vk0 * 2) =
-          make_uint2(__builtin_amdgcn_perm(w1, w0, sel), __builtin_amdgcn_perm(w3, w2, sel));
-    }
+  load_owned<D>(qf, a.q + b * a.sqb + hd * a.sqh, a.sqs, S, qi, h);
+  const TileDma<D, R> kd(a.k + b * a.skb + hd * a.skh, a.sks, S, wave, lane);
+  const TileDma<D, R> vd(a.v + b * a.svb + hd * a.svh, a.svs, S, wave, lane);
+  const int last = qb * kAttnRows + kAttnRows < S ? qb * kAttnRows + kAttnRows : S;
+  const int steps = (last + R - 1) / R;
+  auto issue = [&](int step) {
+    const uint32_t st = lds0 + (step % kAttnStages) * 2 * T::BYTES;
+    kd.issue(st, step * R, wave);
+    vd.issue(st + T::BYTES, step * R, wave);
   };
 
   float m = -INFINITY, l = 0.0f;
   v16f_a o[D / 32];
 #pragma unroll
   for (int dt = 0; dt < D / 32; ++dt) o[dt] = v16f_a{};
-
-  const int last_key = (q0 + BM - 1 < S - 1) ? q0 + BM - 1 : S - 1;
-  const int nkb = last_key / BN + 1;
-  gload(0);
-  lstore(0);
-  if (nkb > 1) gload(1);
-  __syncthreads();
-  for (int kb = 0; kb < nkb; ++kb) {
-    const uint8_t* sk = sk2[kb & 1];
-    const uint8_t* sv = sv2[kb & 1];
-    const int k0 = kb * BN;
-    if (k0 <= qw0 + 31) {  // else the block lies above this wavefront's diagonal
-
-      // S^T for two 32-key tiles: lane holds keys k0 + 32 kt + 8 (e / 4) + 4 hh + e % 4
-      v16f_a st[KT];
+  issue(0);
+  for (int step = 0; step < steps; ++step) {
+    dma_wait_barrier<0>();
+    if (step + 1 < steps) issue(step + 1);
+    const int key0 = step * R;
+    if (key0 > qw0 + 31) continue;  // above this wavefront's diagonal
+    const uint8_t* kt = smem + (step % kAttnStages) * 2 * T::BYTES;
+    const uint8_t* vt = kt + T::BYTES;
+    // S^T: lane holds keys key0 + 32 t + 8 (e / 4) + 4 h + e % 4 of its query
+    v16f_a st[KT];
 #pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        st[kt] = v16f_a{};
+    for (int t = 0; t < KT; ++t) {
+      st[t] = v16f_a{};
 #pragma unroll
-        for (int s = 0; s < D / 16; ++s) {
-          const v8bf_a kf = as_v8bf(*reinterpret_cast<const uint4*>(
-              sk + (32 * kt + l32) * KP + (16 * s + 8 * hh) * 2));
-          st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], st[kt], 0, 0, 0);
-        }
-      }
-      const bool diag = k0 + BN - 1 > qw0;  // some key of the block lies past some query
-      float mx = -INFINITY;
-      if (diag) {
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int key = k0 + 32 * kt + 8 * (e / 4) + 4 * hh + (e % 4);
-            if (key > qi) st[kt][e] = -INFINITY;
-          }
-      }
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, st[kt][e]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-      // the running max in base-2 units (scale * log2 e > 0 commutes with max)
-      const float mnew = fmaxf(m, mx * a.scale_log2);
-      const float mref = mnew == -INFINITY ? 0.0f : mnew;  // a row with no key yet
-      const float alpha = __builtin_amdgcn_exp2f(m - mref);
-      float ps = 0.0f;
-      uint4 pf[KT][2];
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        float p[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][e], a.scale_log2, -mref));
-          ps = ps + p[e];
-        }
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-          pf[kt][s2] = make_uint4(bf16x2_of(p[8 * s2], p[8 * s2 + 1]),
-                                  bf16x2_of(p[8 * s2 + 2], p[8 * s2 + 3]),
-                                  bf16x2_of(p[8 * s2 + 4], p[8 * s2 + 5]),
-                                  bf16x2_of(p[8 * s2 + 6], p[8 * s2 + 7]));
-      }
-      ps = ps + __shfl_xor(ps, 32, kWave);
-      l = l * alpha + ps;
-      m = mnew;
-      // rescale only when some query's running max grew (alpha == 1 exactly otherwise:
-      // exp2(0) = 1), which after the first blocks is rare
-      const bool rescale = __any(alpha != 1.0f);
-#pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt) {
-        if (rescale) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) o[dt][e] = o[dt][e] * alpha;
-        }
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2) {
-            const uint8_t* row = sv + (32 * dt + l32) * VP + (32 * kt + 16 * s2 + 4 * hh) * 2;
-            const uint2 lo = *reinterpret_cast<const uint2*>(row);
-            const uint2 hi = *reinterpret_cast<const uint2*>(row + 16);
-            const v8bf_a vf = as_v8bf(make_uint4(lo.x, lo.y, hi.x, hi.y));
-            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, as_v8bf(pf[kt][s2]), o[dt], 0, 0,
-                                                            0);
-          }
-      }
+      for (int s = 0; s < D / 16; ++s)
+        st[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(kt, 32 * t, s, lane), qf[s],
+                                                        st[t], 0, 0, 0);
     }
-    // block kb + 1 (in registers since the last iteration) goes to the other buffer, whose
-    // reads all ended before the last barrier; block kb + 2's loads go out
-    if (kb + 1 < nkb) {
-      lstore((kb + 1) & 1);
-      if (kb + 2 < nkb) gload(kb + 2);
+    if (key0 + R - 1 > qw0) {  // some key of the step lies past some query
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (key0 + 32 * t + 8 * (e / 4) + 4 * h + (e % 4) > qi) st[t][e] = -INFINITY;
     }
-    __syncthreads();
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, st[t][e]);
+    mx = half_max(mx);
+    // the running max in base-2 units (scale * log2 e > 0 commutes with max)
+    const float mnew = fmaxf(m, mx * a.scale_log2);
+    const float mref = mnew == -INFINITY ? 0.0f : mnew;  // a row with no key yet
+    const float alpha = __builtin_amdgcn_exp2f(m - mref);
+    m = mnew;
+    // rescale only when some query's running max grew (alpha == 1 exactly otherwise:
+    // exp2(0) = 1), which after the first steps is rare
+    if (__any(alpha != 1.0f)) {
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[dt][e] = o[dt][e] * alpha;
+    }
+    float ps = 0.0f;
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      float p[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[t][e], a.scale_log2, -mref));
+        ps = ps + p[e];
+      }
+      uint4 pf[2];
+      pack16(pf, p);
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              col_frag<D>(vt, 32 * t + 16 * s2, dt, lane), frag_of(pf[s2]), o[dt], 0, 0, 0);
+    }
+    l = l * alpha + half_sum(ps);
   }
 
-  // o[dt][e] = O[qi][32 dt + 8 (e / 4) + 4 hh + e % 4] * l
   if (qi < S) {
-    const float inv = 1.0f / l;
-    uint16_t* orow = a.o + b * a.sob + h * a.soh + static_cast<int64_t>(qi) * a.sos;
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int d0 = 32 * dt + 8 * r + 4 * hh;
-        *reinterpret_cast<uint2*>(orow + d0) =
-            make_uint2(bf16x2_of(o[dt][4 * r] * inv, o[dt][4 * r + 1] * inv),
-                       bf16x2_of(o[dt][4 * r + 2] * inv, o[dt][4 * r + 3] * inv));
-      }
-    if (hh == 0) a.lse[bh * S + qi] = (m + __log2f(l)) * 0.69314718055994531f;
+    store_owned<D>(a.o + b * a.sob + hd * a.soh + static_cast<int64_t>(qi) * a.sos, o, 1.0f / l, h);
+    if (h == 0) a.lse[bh * a.S + qi] = (m + __log2f(l)) * 0.69314718055994531f;
   }
 }
 
@@ -281,13 +190,13 @@ extern "C" int rk_attention_forward(const uint16_t* q, int64_t sqb, int64_t sqh,
   if ((rows * sqs + D) * 2 >= (int64_t{1} << 31) || (rows * sks + D) * 2 >= (int64_t{1} << 31) ||
       (rows * svs + D) * 2 >= (int64_t{1} << 31))
     return fail(RK_ERR_UNSUPPORTED, "sequence extent exceeds 2^31 bytes per head");
-  if (B * H > 0x7fffffff || (S + kAttnBM - 1) / kAttnBM > 0x7fffffff)
+  const int64_t blocks = B * H * ((S + kAttnRows - 1) / kAttnRows);
+  if (B * H > 0x7fffffff || blocks >= (int64_t{1} << 24))  // 2^32 threads
     return fail(RK_ERR_ARG, "grid too large");
   AttnArgs a{q, k, v, sqb, sqh, sqs, skb, skh, sks, svb, svh, svs, o, sob, soh, sos, lse,
              B, H, S, scale * 1.4426950408889634f};
-  const dim3 grid(static_cast<unsigned>((S + kAttnBM - 1) / kAttnBM),
-                  static_cast<unsigned>(B * H));
+  const dim3 grid(static_cast<unsigned>(blocks));
   if (D == 64) attn_fwd_kernel<64, 64><<<grid, 256, 0, as_stream(stream)>>>(a);
-  else attn_fwd_kernel<128, 32><<<grid, 256, 0, as_stream(stream)>>>(a);
+  else attn_fwd_kernel<128, 64><<<grid, 256, 0, as_stream(stream)>>>(a);
   return launch_status("attention_forward");
 }

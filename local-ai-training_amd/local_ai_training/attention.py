@@ -4,9 +4,13 @@ The reference attends with ``F.scaled_dot_product_attention(q, k, v, is_causal=T
 (``model.py:117-123``). Here the forward is ``rk_attention_forward`` (flash form on the bf16
 MFMA, ``csrc/rk_attention.hip``), which writes the output and the per-query log-sum-exp in
 the form torch's memory-efficient attention forward does; the backward is
-``rk_attention_backward`` (``csrc/rk_attention_bwd.hip``) on those two tensors. torch's
-memory-efficient backward (which adds its float32 dq by atomics, in an order that varies)
-stays for extents the HIP kernels' 32-bit offsets do not reach.
+``rk_attention_backward`` (``csrc/rk_attention_bwd.hip``) at head size 128 (165 us at B 8,
+H 16, S 1024 against 293 us for torch's memory-efficient backward, which adds its float32 dq by
+atomics in an order that varies). At head size 64 it stays torch's memory-efficient backward,
+called on the forward's two tensors: the HIP kernels were faster there too (70 against 131 us
+at B 32, H 8, S 512), but any other rounding of those gradients moves the loss of the 25M
+training step by up to 1e-3 within four steps (through the stochastic rounding and the update's
+thresholds), above the 5e-4 that step is held to (``perf/cases.py``).
 
 Supported: bfloat16 GPU q, k, v [B, H, S, D] with D 64 or 128, unit feature stride,
 16-byte aligned storage and strides that are multiples of 8 elements, no attention mask,
@@ -60,16 +64,17 @@ def attention_supported(q: Tensor, k: Tensor, v: Tensor) -> bool:
 
 
 def _backward_fits(tensors: tuple[Tensor, ...]) -> bool:
-    """The limits of ``rk_attention_backward``'s 32-bit offsets: one head's rows up to the
-    padded length within 2^31 bytes of bf16, and its two float32 statistics per padded row."""
+    """What ``rk_attention_backward`` takes: head size 128, and the limits of its 32-bit
+    offsets (one head's rows up to the padded length within 2^31 bytes of bf16, and all rows'
+    two float32 statistics)."""
     b, h, s, d = tensors[0].shape
     padded = -(-s // 128) * 128
-    return (8 * b * h * padded < 2**31 and padded // 128 <= 65535
+    return (d == 128 and 8 * b * h * padded < 2**31
             and all(((padded + 64) * t.stride(2) + d) * 2 < 2**31 for t in tensors))
 
 
 class CausalAttentionFn(torch.autograd.Function):
-    """o = causal softmax(q k^T / sqrt(D)) v: HIP forward and backward."""
+    """o = causal softmax(q k^T / sqrt(D)) v: HIP forward, HIP backward at head size 128."""
 
     @staticmethod
     def forward(ctx, q: Tensor, k: Tensor, v: Tensor) -> Tensor:
