@@ -91,12 +91,9 @@ __device__ __forceinline__ float load_elem(const void* base, int64_t idx) {
   }
 }
 
-// Loads one 16-byte vector (Vec<DT>::N elements) at element index idx (must be
-// 16-byte aligned) and widens it to fp32.
+// One 16-byte vector (Vec<DT>::N elements) widened to fp32.
 template <int DT>
-__device__ __forceinline__ void load_vec16(const void* base, int64_t idx, float* out) {
-  const uint4 raw = *reinterpret_cast<const uint4*>(
-      static_cast<const char*>(base) + idx * (DT == RK_F32 ? 4 : 2));
+__device__ __forceinline__ void widen_vec16(const uint4& raw, float* out) {
   if constexpr (DT == RK_F32) {
     out[0] = __uint_as_float(raw.x);
     out[1] = __uint_as_float(raw.y);
@@ -110,6 +107,14 @@ __device__ __forceinline__ void load_vec16(const void* base, int64_t idx, float*
       out[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
     }
   }
+}
+
+// Loads one 16-byte vector at element index idx (must be 16-byte aligned) and widens it.
+template <int DT>
+__device__ __forceinline__ void load_vec16(const void* base, int64_t idx, float* out) {
+  widen_vec16<DT>(*reinterpret_cast<const uint4*>(static_cast<const char*>(base) +
+                                                  idx * (DT == RK_F32 ? 4 : 2)),
+                  out);
 }
 
 // tanh(u) = 1 - 2 / (exp(2u) + 1) from the hardware exp2 and reciprocal (v_exp_f32,

@@ -12,6 +12,12 @@
 //   SRC_RMSNORM   x * rsqrt(mean x^2 + eps) * w,          int8_fused.py:14-39
 //   SRC_GELU      tanh-GELU(x),                           int8_fused.py:58-84
 //   SRC_TRANSPOSE [B,H,S,D] read as [B*S, H*D],           int8_fused.py:103-131
+//
+// Stochastic rounding is bound by Philox: 17 wide multiplies per value (v_mad_u64_u32, two issue
+// slots each) beside 29 other instructions, 252 cycles per 64 values and SIMD, 54 us for
+// 16384 x 2048. Measured 62.8 us with the uniform formed and the quotient's flags kept per
+// value, 59.3 us through sr_fast (rk_rowquant.h); 8192 x 6144 94 -> 87 us, 8192 x 2048 float32
+// with its bf16 copy (stored two bytes at a time before) 48 -> 43 us.
 #include "rk_common.h"
 #include "rk_rowquant.h"
 
@@ -67,7 +73,7 @@ __device__ __forceinline__ void load_chunk(const QuantArgs& a, int64_t row, int6
   constexpr int V = Vec<DT>::N;
   if constexpr (SRC == SRC_PLAIN) {
     if (a.nparts > 0) {
-      const int64_t p = e0 / a.part_cols;
+      const int p = (e0 >= a.part_cols) + (e0 >= 2 * a.part_cols);  // at most three parts
       const void* base = p == 0 ? a.xp[0] : (p == 1 ? a.xp[1] : a.xp[2]);
       const int64_t idx = row * a.sxm + (e0 - p * a.part_cols);
       if (VEC || (a.vec_ok && e0 + V <= a.K)) {
@@ -90,6 +96,22 @@ __device__ __forceinline__ void load_chunk(const QuantArgs& a, int64_t row, int6
   }
 }
 
+// The 16-byte vector at columns e0 .. of a row (vector loads legal, the chunk inside the row).
+template <int DT, int SRC>
+__device__ __forceinline__ uint4 load_raw(const QuantArgs& a, int64_t row, int64_t e0) {
+  constexpr int ES = DT == RK_F32 ? 4 : 2;
+  const void* base = a.x;
+  int64_t idx;
+  if (SRC == SRC_PLAIN && a.nparts > 0) {
+    const int p = (e0 >= a.part_cols) + (e0 >= 2 * a.part_cols);
+    base = p == 0 ? a.xp[0] : (p == 1 ? a.xp[1] : a.xp[2]);
+    idx = row * a.sxm + (e0 - p * a.part_cols);
+  } else {
+    idx = src_offset<DT, SRC>(a, row, e0);
+  }
+  return *reinterpret_cast<const uint4*>(static_cast<const char*>(base) + idx * ES);
+}
+
 // Row transform applied to a raw value at column e (row_factor = rsqrt for rmsnorm).
 template <int DT, int SRC>
 __device__ __forceinline__ float transform(const QuantArgs& a, float x, int64_t e,
@@ -110,8 +132,17 @@ __device__ __forceinline__ float transform(const QuantArgs& a, float x, int64_t 
 
 template <int DT>
 __device__ __forceinline__ void store_bf16_chunk(uint16_t* dst, int64_t e0, int64_t K,
-                                                 const float* v) {
+                                                 const float* v, bool vec) {
   constexpr int V = Vec<DT>::N;
+  if (vec && e0 + V <= K) {  // one store of the V values
+    uint32_t w[V / 2];
+#pragma unroll
+    for (int i = 0; i < V / 2; ++i)
+      w[i] = f32_to_bf16(v[2 * i]) | (static_cast<uint32_t>(f32_to_bf16(v[2 * i + 1])) << 16);
+    if constexpr (V == 8) *reinterpret_cast<uint4*>(dst + e0) = make_uint4(w[0], w[1], w[2], w[3]);
+    else *reinterpret_cast<uint2*>(dst + e0) = make_uint2(w[0], w[1]);
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < V; ++i)
     if (e0 + i < K) dst[e0 + i] = f32_to_bf16(v[i]);
@@ -125,23 +156,36 @@ __device__ __forceinline__ void quant_store_chunk(const QuantArgs& a, uint32_t c
                                                   const float* y, float s, float r,
                                                   int8_t* qrow, bool vec_store) {
   constexpr int V = Vec<DT>::N;
-  float t[V], u[V];
-  bool exact = false;
+  float t[V];
+  if constexpr (SR) {
+    // counter = (row_offset + m) * K + k, wrapped to 32 bits like the int32 offsets
+    // of int8_matmul.py:143
+    uint32_t word[V];
+    float worst = 0.0f;
 #pragma unroll
-  for (int i = 0; i < V; ++i) {
-    u[i] = 0.0f;
-    if constexpr (SR) {
-      // counter = (row_offset + m) * K + k, wrapped to 32 bits like the int32 offsets
-      // of int8_matmul.py:143
-      u[i] = uniform_from_word(philox_word0(ctr_row + static_cast<uint32_t>(e0 + i), key));
+    for (int i = 0; i < V; ++i) {
+      word[i] = philox_word0(ctr_row + static_cast<uint32_t>(e0 + i), key);
+      t[i] = sr_fast(y[i], r, word[i], worst);
     }
-    t[i] = round_fast<SR>(y[i], r, u[i], exact);
-  }
-  if (exact) {
-    // a value of this lane's chunk lies within the margin of a rounding boundary (or is
-    // not finite): round the chunk through round_quotient, which divides where needed
 #pragma unroll
-    for (int i = 0; i < V; ++i) t[i] = round_quotient<SR>(y[i], s, r, u[i]);
+    for (int i = 0; i < V; ++i) t[i] = floorf(t[i]);
+    if (worst > 0.5f - kSrAmbiguity) {
+      // a value of this lane's chunk lies within the margin of an integer: round the chunk
+      // through round_quotient, which divides where needed
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        t[i] = round_quotient<true>(y[i], s, r, uniform_from_word(word[i]));
+    }
+  } else {
+    bool exact = false;
+#pragma unroll
+    for (int i = 0; i < V; ++i) t[i] = round_fast<false>(y[i], r, 0.0f, exact);
+    if (exact) {
+      // a value of this lane's chunk lies within the margin of a rounding boundary (or is
+      // not finite)
+#pragma unroll
+      for (int i = 0; i < V; ++i) t[i] = round_quotient<false>(y[i], s, r, 0.0f);
+    }
   }
   int qi[V];
 #pragma unroll
@@ -212,6 +256,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
   int8_t* qrow = a.q + row * a.ldq;
   const bool vec_store = (a.ldq % V) == 0 && ((reinterpret_cast<uintptr_t>(a.q) % V) == 0);
   uint16_t* xbrow = (SRC == SRC_PLAIN && a.xb) ? a.xb + row * a.ldxb : nullptr;
+  const bool xb_vec = a.ldxb % V == 0 && reinterpret_cast<uintptr_t>(a.xb) % (2 * V) == 0;
   PhiloxKey key{};
   if constexpr (SR) {
     uint32_t k0 = a.key0, k1 = a.key1;
@@ -229,15 +274,37 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
     // Register-resident row (or row slice): one HBM read.
     const int c0 = slice * NC;  // this wavefront's first chunk
     float xr[NC][V];
+    if constexpr (VEC) {
+      // every chunk's load in flight before the first is used; lanes past the row read its
+      // first vector (in bounds) and take zeros
+      uint4 raw[NC];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int64_t e0 = (c0 + c) * SPAN + lane0;
-      if (c0 + c < nchunks && (!VEC || e0 < a.K)) {
-        load_chunk<DT, SRC, VEC>(a, row, e0, xr[c]);
-        if (xbrow && e0 < a.K) store_bf16_chunk<DT>(xbrow, e0, a.K, xr[c]);
-      } else {
+      for (int c = 0; c < NC; ++c) {
+        const int64_t e0 = (c0 + c) * SPAN + lane0;
+        raw[c] = load_raw<DT, SRC>(a, row, e0 < a.K ? e0 : 0);
+      }
 #pragma unroll
-        for (int i = 0; i < V; ++i) xr[c][i] = 0.0f;
+      for (int c = 0; c < NC; ++c) {
+        if ((c0 + c) * SPAN + lane0 >= a.K) raw[c] = make_uint4(0, 0, 0, 0);
+        widen_vec16<DT>(raw[c], xr[c]);
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int64_t e0 = (c0 + c) * SPAN + lane0;
+        if (c0 + c < nchunks) {
+          load_chunk<DT, SRC, VEC>(a, row, e0, xr[c]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < V; ++i) xr[c][i] = 0.0f;
+        }
+      }
+    }
+    if (xbrow) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int64_t e0 = (c0 + c) * SPAN + lane0;
+        if (e0 < a.K) store_bf16_chunk<DT>(xbrow, e0, a.K, xr[c], xb_vec);
       }
     }
     float row_factor = 1.0f;
@@ -310,7 +377,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
       if (e0 >= a.K) break;
       float v[V];
       load_chunk<DT, SRC, VEC>(a, row, e0, v);
-      if (xbrow) store_bf16_chunk<DT>(xbrow, e0, a.K, v);
+      if (xbrow) store_bf16_chunk<DT>(xbrow, e0, a.K, v, xb_vec);
       transform_chunk<DT, SRC, VEC>(a, e0, v, row_factor);
       quant_store_chunk<DT, SR, VEC>(a, ctr_row, key, e0, v, s, r, qrow, vec_store);
     }

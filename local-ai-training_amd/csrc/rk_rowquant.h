@@ -28,6 +28,26 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 // div_rn) and rounds that.
 constexpr float kAmbiguity = 0.000244140625f;
 
+// The stochastic fast path: v close to RN(Y + u), Y = RN(y / s), u the uniform of the random
+// word w, without the division and without forming u (five instructions where the exact form
+// takes ten): |float(int(w))| differs from float(w < 0 ? ~w : w) by at most one in 2^31 before
+// rounding, and the product with 2^-31 and the add round once. Errors of v against RN(Y + u),
+// for |y / s| <= 127.00002 (r = RN(1 / s)): y * r, 127 * 2^-23; the rounding of Y, 2^-18; u,
+// 2^-24; the two adds, 2^-18 each below 128 (twice that above, where the clamp decides).
+// Together under 2^-15, so outside kSrAmbiguity = 2^-14 of an integer floor(v) is
+// floor(RN(Y + u)). `worst` collects max |fract(v) - 1/2| over a group; only a group with
+// worst > 1/2 - kSrAmbiguity is redone through round_quotient. Non-finite values need no flag:
+// a NaN y / s gives NaN both ways, and a row with an infinite absmax has r = 0, so its finite
+// values give floor(u) = 0 both ways.
+constexpr float kSrAmbiguity = 0.00006103515625f;
+
+__device__ __forceinline__ float sr_fast(float y, float r, uint32_t w, float& worst) {
+  const float k = fabsf(static_cast<float>(static_cast<int32_t>(w)));
+  const float v = __builtin_fmaf(k, __uint_as_float(0x2FFFFFFFu), y * r);
+  worst = fmaxf(worst, fabsf(__builtin_amdgcn_fractf(v) - 0.5f));
+  return v;
+}
+
 // The fast path of round_quotient alone: the rounded value from ya = y * r, with `exact`
 // set (never cleared) where that value may differ from the one computed from y / s (the
 // same test as round_quotient's). Callers round a group of values this way and redo the
