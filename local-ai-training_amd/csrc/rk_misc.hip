@@ -42,6 +42,29 @@ __global__ void unpack_kernel(const uint8_t* packed, int64_t n, int mc, int8_t* 
   }
 }
 
+// The same 16 bytes per thread (aligned pointers): at 46 M weights, 8.4 of the 26 us a byte
+// per thread took; the last n % 16 bytes go to the first threads.
+__global__ __launch_bounds__(256) void unpack_vec_kernel(const uint8_t* packed, int64_t n, int mc,
+                                                         int8_t* code, int8_t* pressure) {
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const uint32_t mc4 = static_cast<uint32_t>(mc) * 0x01010101u;
+  for (int64_t i = first; i < n / 16; i += static_cast<int64_t>(gridDim.x) * 256) {
+    const uint4 w = reinterpret_cast<const uint4*>(packed)[i];
+    if (code)
+      reinterpret_cast<uint4*>(code)[i] =
+          make_uint4(decode4(w.x, mc4), decode4(w.y, mc4), decode4(w.z, mc4), decode4(w.w, mc4));
+    if (pressure)
+      reinterpret_cast<uint4*>(pressure)[i] =
+          make_uint4(decode4(w.x >> 4, 0x07070707u), decode4(w.y >> 4, 0x07070707u),
+                     decode4(w.z >> 4, 0x07070707u), decode4(w.w >> 4, 0x07070707u));
+  }
+  const int64_t t = n / 16 * 16 + first;
+  if (t < n) {
+    if (code) code[t] = static_cast<int8_t>((packed[t] & 15) - mc);
+    if (pressure) pressure[t] = static_cast<int8_t>((packed[t] >> 4) - 7);
+  }
+}
+
 // 64x64 tiles through LDS: packed[n, k] -> codeT[k, n].
 __global__ __launch_bounds__(256) void unpack_transpose_kernel(const uint8_t* packed,
                                                                int64_t ldp, int mc,
@@ -221,8 +244,15 @@ extern "C" int rk_unpack(const uint8_t* packed, int64_t n, int max_code, int8_t*
   if (n < 0) return fail(RK_ERR_ARG, "negative size");
   if (n == 0) return RK_OK;
   if (!packed) return fail(RK_ERR_ARG, "null packed state");
-  unpack_kernel<<<flat_grid(n, 1), 256, 0, as_stream(stream)>>>(packed, n, max_code, code,
-                                                                 pressure);
+  // (a null code or pressure counts as aligned)
+  if (aligned16(packed) && aligned16(code) && aligned16(pressure) && max_code >= 0 &&
+      max_code <= 15) {
+    unpack_vec_kernel<<<flat_grid(n, 16), 256, 0, as_stream(stream)>>>(packed, n, max_code, code,
+                                                                       pressure);
+  } else {
+    unpack_kernel<<<flat_grid(n, 1), 256, 0, as_stream(stream)>>>(packed, n, max_code, code,
+                                                                  pressure);
+  }
   return launch_status("unpack");
 }
 

@@ -55,9 +55,17 @@ __global__ __launch_bounds__(256) void ratchet_update_z_kernel(
 
 // Mean of rows values with one 256-thread block, in a fixed order: thread t adds rows t,
 // t + 256, ... in order, then a halving tree (t += t + w for w = 128 .. 1). Thread 0 gets it.
+// Eight rows' loads are in flight before their adds (one at a time, 8192 rows took 10 us).
 __device__ __forceinline__ float block_mean_256(const float* x, int64_t rows, float* part) {
   float acc = 0.0f;
-  for (int64_t r = threadIdx.x; r < rows; r += 256) acc = acc + x[r];
+  for (int64_t r = threadIdx.x; r < rows; r += 8 * 256) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = x[r + 256 * j < rows ? r + 256 * j : r];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (r + 256 * j < rows) acc = acc + v[j];
+  }
   part[threadIdx.x] = acc;
   __syncthreads();
   for (int w = 128; w >= 1; w >>= 1) {
