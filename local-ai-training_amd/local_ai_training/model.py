@@ -120,16 +120,23 @@ class KVCache:
         self._mask: Tensor | None = None
         self.step_buffers: dict[str, Tensor] = {}  # fixed-shape work buffers of a step
 
-    def buffers(self, layer: int, like: Tensor) -> tuple[Tensor, Tensor]:
+    def buffers(self, layer: int, like: Tensor, written: int = 0) -> tuple[Tensor, Tensor]:
         """The layer's key/value buffers, allocated on first use in the cache dtype
         (``like``'s when none was given) and kept from then on (later steps convert to
-        their dtype, so keys written by a prefill are never dropped)."""
+        their dtype, so keys written by a prefill are never dropped). New buffers are zero,
+        but for the first ``written`` positions, which the caller writes at once."""
         if self.keys[layer] is None:
             dtype = self.dtype or like.dtype
             shape = (self.batch, self.n_head, self.max_len, self.head_size)
-            self.keys[layer] = torch.zeros(shape, dtype=dtype, device=self.device)
-            self.values[layer] = torch.zeros(shape, dtype=dtype, device=self.device)
+            for side in (self.keys, self.values):
+                side[layer] = torch.empty(shape, dtype=dtype, device=self.device)
+                side[layer][:, :, written:].zero_()
         return self.keys[layer], self.values[layer]
+
+    def stores_bf16(self, layer: int) -> bool:
+        """Whether the layer's keys and values are (or will be) stored as bfloat16."""
+        kept = self.keys[layer]
+        return (self.dtype if kept is None else kept.dtype) == torch.bfloat16
 
     def decode_mask(self, dtype: torch.dtype) -> Tensor:
         """Additive mask [1, 1, 1, max_len] for a one-token step at position ``pos``:
@@ -246,14 +253,23 @@ class CausalSelfAttention(nn.Module):
         """``residual``: return residual + attention output (int8 projection: added in the
         GEMM epilogue)."""
         batch_size, sequence_length, channels = inputs.shape
+        projection_kw = {}
         if inputs_int8 is not None:
             # Under bf16 autocast the attention casts q, k, v to bf16 (and their gradients
             # back): take the GEMM's bf16 result directly instead (the same values; no cast
             # kernels). The layer returns the three chunks itself, so their gradients reach
             # its backward separately and are read there in place (no concatenation).
+            # The same holds without autocast where nothing is differentiated and the keys and
+            # values are cached in bf16: the float32 result would only be narrowed again.
             kw = {"split": 3} if self.split_qkv_grad else {}
+            out_dtype = _autocast_bf16(inputs)
+            if (out_dtype is None and cache is not None and inputs.dtype == torch.float32
+                    and not torch.is_grad_enabled() and cache.stores_bf16(layer)
+                    and _is_int8(self.projection)):
+                out_dtype = torch.bfloat16
+                projection_kw = {"out_dtype": inputs.dtype}  # the layer's output stays float32
             qkv = self.qkv(inputs, inputs_int8=inputs_int8, inputs_scale=inputs_scale,
-                           out_dtype=_autocast_bf16(inputs), **kw)
+                           out_dtype=out_dtype, **kw)
         else:
             qkv = self.qkv(inputs)
         query, key, value = qkv if isinstance(qkv, tuple) else qkv.chunk(3, dim=-1)
@@ -270,7 +286,7 @@ class CausalSelfAttention(nn.Module):
         if _is_int8(self.projection):
             attn_int8, attn_scale, dummy = FusedTransposeQuantizeFn.apply(attended)
             return self.projection(dummy, inputs_int8=attn_int8, inputs_scale=attn_scale,
-                                   residual=residual)
+                                   residual=residual, **projection_kw)
         joined = attended.transpose(1, 2).contiguous().view(batch_size, sequence_length, channels)
         out = self.projection(joined)
         return out if residual is None else residual + out
@@ -281,7 +297,10 @@ class CausalSelfAttention(nn.Module):
         values. ``decode``: one token at the device-side position ``cache.pos``, attending
         over the whole buffer under a mask (fixed shapes); otherwise a prompt of S tokens
         written at the host-side ``cache.length`` (causal among themselves)."""
-        keys, values = cache.buffers(layer, k)
+        start, length = cache.length, q.shape[2]
+        keys, values = cache.buffers(layer, k,
+                                     length if not decode and start == 0
+                                     and length <= cache.max_len else 0)
         out_dtype = q.dtype
         if keys.dtype != q.dtype:
             q, k, v = q.to(keys.dtype), k.to(keys.dtype), v.to(keys.dtype)
@@ -290,7 +309,6 @@ class CausalSelfAttention(nn.Module):
             values.index_copy_(2, cache.pos, v)
             out = _attend(q, keys, values, attn_mask=cache.decode_mask(q.dtype))
             return out.to(out_dtype)
-        start, length = cache.length, q.shape[2]
         end = start + length
         if end > cache.max_len:
             raise ValueError("KV cache is full")
@@ -324,7 +342,13 @@ class FeedForward(nn.Module):
         """``residual``: return residual + feed-forward output (int8 contraction without
         active dropout: added in the GEMM epilogue)."""
         int8_contract = _is_int8(self.contract)
-        bf16_out = _autocast_bf16(inputs) if int8_contract and self.bf16_expand else None
+        bf16_out = None
+        if int8_contract and self.bf16_expand:
+            bf16_out = _autocast_bf16(inputs)
+            # without gradients the GELU prologue reads the bf16 result too (the same values)
+            if (bf16_out is None and inputs.is_cuda and inputs.dtype == torch.float32
+                    and not torch.is_grad_enabled()):
+                bf16_out = torch.bfloat16
         kw = {"out_dtype": bf16_out} if bf16_out is not None else {}
         if inputs_int8 is not None:
             expanded = self.expand(inputs, inputs_int8=inputs_int8, inputs_scale=inputs_scale,
