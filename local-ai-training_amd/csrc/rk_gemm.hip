@@ -546,22 +546,13 @@ void int8_gemm_m32_kernel(GemmArgs g) {
 //    lanes) then touch 16 distinct 16-byte bank groups.
 // The row scales (and column scales) of each tile go to a double-buffered LDS area by the
 // same DMA, ahead of the tile's first k-step, so the epilogue reads them with no vector
-// memory wait. The epilogue stages the bf16 results in LDS, 32 rows per round, so every
+// memory wait. The epilogue stages the bf16 results in LDS, 64 rows per round, so every
 // store writes 16 bytes of 32-lane-contiguous 512-byte rows (stores straight from the MFMA
 // layout scatter 8 bytes over 32 rows per instruction and cost 18 of 45 us at
 // 16384 x 2048 x 512). Out-of-range columns are stored to an offset past the output
 // descriptor (2^31, dropped by the hardware) instead of behind a branch. Tiles are walked in
 // groups of 8 row tiles (n-major inside a group), so the 32 tiles an XCD runs at once
 // share 8 A panels and 4 B panels in its L2 (8192^3: 626 -> 534 us against row-major).
-//
-// The 32-byte k halves are software-pipelined: a half's fragments are read from LDS before the
-// products of the half before it, so that the LDS (12 KB per wavefront and half, about as long
-// as the products at the full LDS rate) works while the matrix pipe does; the wait for the
-// next stage therefore sits between a step's halves, and a fourth stage gives the loads their
-// two steps back. Against reading each half just before its products, on one box (us): 8192 x
-// 6144 x 2048 bf16 143 -> 132, 8192 x 8192 x 2048 float32 184 -> 174, 16384 x 8192 x 512
-// float32 181 -> 175, 8192^3 565 -> 531 (2.07 POP/s; the library's int8 product of that shape
-// reaches 2.0 on this card); with three stages 136, 178, 191 and 530.
 //
 // Synchronization per k-step: each wavefront waits for its own DMA loads of the stage
 // (vmcnt, and lgkmcnt(0): the LDS write of an LDS-DMA load is tracked on the LDS counter, and
@@ -573,9 +564,9 @@ void int8_gemm_m32_kernel(GemmArgs g) {
 // ---------------------------------------------------------------------------
 typedef unsigned int u32x2_v __attribute__((ext_vector_type(2)));
 
-constexpr int kPipeBM = 256, kPipeBN = 256, kPipeBK = 64, kPipeStages = 4;
-// epilogue staging: 32 rows of 256 bf16 at a 520-byte pitch (rows 2 banks apart)
-constexpr int kEPitch = 520, kERows = 32;
+constexpr int kPipeBM = 256, kPipeBN = 256, kPipeBK = 64, kPipeStages = 3;
+// epilogue staging: 64 rows of 256 bf16 at a 520-byte pitch (rows 2 banks apart)
+constexpr int kEPitch = 520, kERows = 64;
 constexpr int kPipeStage = (kPipeBM + kPipeBN) * kPipeBK;  // 32 KB
 constexpr int kPipeScales = 2 * 2 * 1024;                  // ls + rs, two tiles
 
@@ -687,79 +678,60 @@ void int8_gemm_pipe_kernel(GemmArgs g, PipeSched p) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = v16i{};
 
-  // One 32-byte k half of a stage: this wavefront's fragments, and the products over them.
-  auto read_half = [&](v4i (&fa)[MI], v4i (&fb)[NJ], int stage, int kh) {
-    const uint8_t* at = smem + stage * STAGE;
-    const uint8_t* bt = at + ASZ;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      if constexpr (BT) {
-        // 16 consecutive k rows of output column `col` per lane (transposing read)
-        const int sl = lane & 15;
-        const int col = brow0 + j * 32 + 16 * ((lane >> 4) & 1) + 8 * (sl & 1);
-        const int r0 = 16 * (h + 2 * kh) + (sl >> 1);  // r0 & 7 == (r0 + 8) & 7
-        const int phys = 16 * ((col >> 4) ^ (2 * (r0 & 7))) + (col & 15);
-        const v2i_t lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(bt + r0 * 256 + phys));
-        const v2i_t hi =
-            __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(bt + (r0 + 8) * 256 + phys));
-        fb[j] = v4i{lo.x, lo.y, hi.x, hi.y};
-      } else {
-        const int rb = brow0 + j * 32 + r32;
-        fb[j] = *reinterpret_cast<const v4i*>(bt + rb * 64 + 16 * ((h + 2 * kh) ^ swz32(rb)));
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int ra = arow0 + i * 32 + r32;
-      fa[i] = *reinterpret_cast<const v4i*>(at + ra * 64 + 16 * ((h + 2 * kh) ^ swz32(ra)));
-    }
-  };
-  auto multiply = [&](const v4i (&fa)[MI], v4i (&fb)[NJ]) {
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      if constexpr (PACKED) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          fb[j][e] = static_cast<int>(decode4(static_cast<uint32_t>(fb[j][e]), g.mc4));
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[j], fa[i], acc[i][j], 0, 0, 0);
-  };
-
-  // The k halves are software-pipelined: the fragments of the next half (of the next step, once
-  // its stage has landed in the middle of this one) are read from LDS before this half's
-  // products, so the LDS and the matrix pipe work at the same time in every wavefront.
-  v4i fa0[MI], fb0[NJ], fa1[MI], fb1[NJ];
-  // waits until the stage of step `next` has landed, `later` stages after it in flight
-  auto land = [&](int later) {
-    if (later >= 2) dma_wait_barrier<4 * CH>();
-    else if (later == 1) dma_wait_barrier<2 * CH>();
-    else dma_wait_barrier<0>();
-  };
   for (int s = 0; s < S - 1 && s < total; ++s) issue();
-  if (total > 0) {
-    land(total - 1 < S - 2 ? total - 1 : S - 2);
-    read_half(fa0, fb0, 0, 0);
-  }
   int ct = 0, ck = 0, cstage = 0;  // consumer: tile ordinal, k-step, stage
   for (int step = 0; step < total; ++step) {
-    read_half(fa1, fb1, cstage, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(fa0, fb0);
+    // this step's loads landed: at most the loads of the (up to S - 2) later steps in
+    // flight (2 CH per step; the scale loads and stores issued after them only make the
+    // wait stricter)
+    const int ahead = total - 1 - step;
+    if (ahead >= S - 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * CH * (S - 2)) & ~0x0F00);
+    else if (ahead == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * CH) & ~0x0F00);
+    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0) & ~0x0F00);
+    asm volatile("s_barrier" ::: "memory");
+    if (step + S - 1 < total) issue();
+
+    const uint8_t* at = smem + cstage * STAGE;
     if (++cstage == S) cstage = 0;
-    if (step + 1 < total) {
-      // stage step + 1 has landed; the stage refilled after the barrier is step - 1's, which
-      // every wavefront has multiplied before it arrived
-      land(total - 2 - step < S - 3 ? total - 2 - step : S - 3);
-      if (step + S - 1 < total) issue();
-      read_half(fa0, fb0, cstage, 0);
-      __builtin_amdgcn_sched_barrier(0);
+    const uint8_t* bt = at + ASZ;
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      v4i fa[MI], fb[NJ];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const int ra = arow0 + i * 32 + r32;
+        fa[i] = *reinterpret_cast<const v4i*>(at + ra * 64 + 16 * ((h + 2 * kh) ^ swz32(ra)));
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        v4i v;
+        if constexpr (BT) {
+          // 16 consecutive k rows of output column `col` per lane (transposing read)
+          const int sl = lane & 15;
+          const int col = brow0 + j * 32 + 16 * ((lane >> 4) & 1) + 8 * (sl & 1);
+          const int r0 = 16 * (h + 2 * kh) + (sl >> 1);  // r0 & 7 == (r0 + 8) & 7
+          const int phys = 16 * ((col >> 4) ^ (2 * (r0 & 7))) + (col & 15);
+          const v2i_t lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(bt + r0 * 256 + phys));
+          const v2i_t hi =
+              __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(bt + (r0 + 8) * 256 + phys));
+          v = v4i{lo.x, lo.y, hi.x, hi.y};
+        } else {
+          const int rb = brow0 + j * 32 + r32;
+          v = *reinterpret_cast<const v4i*>(bt + rb * 64 + 16 * ((h + 2 * kh) ^ swz32(rb)));
+        }
+        if constexpr (PACKED) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[e] = static_cast<int>(decode4(static_cast<uint32_t>(v[e]), g.mc4));
+        }
+        fb[j] = v;
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[j], fa[i], acc[i][j], 0, 0, 0);
     }
-    multiply(fa1, fb1);
     if (++ck < nk) continue;
 
     // Epilogue of tile ct: C = bf16((acc * ls) * rs), rows m = arow0 + 32 i + lane % 32,
@@ -785,38 +757,40 @@ void int8_gemm_pipe_kernel(GemmArgs g, PipeSched p) {
       uint8_t* stg = smem + S * STAGE + kPipeScales;
       const int wm = wave & 1;
 #pragma unroll
-      for (int round = 0; round < 8; ++round) {
-        if (wm == (round >> 2)) {
-          const int i = round & 3;
+      for (int round = 0; round < 4; ++round) {
+        if (wm == (round >> 1)) {
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) {
+          for (int ii = 0; ii < 2; ++ii) {
+            const int i = 2 * (round & 1) + ii;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int nl = brow0 + 32 * j + 8 * q + 4 * h;
-              float4 rs4 = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-              if constexpr (HAS_RS) rs4 = *reinterpret_cast<const float4*>(sc + 1024 + nl * 4);
-              float v0 = static_cast<float>(acc[i][j][4 * q]) * lsv[i];
-              float v1 = static_cast<float>(acc[i][j][4 * q + 1]) * lsv[i];
-              float v2 = static_cast<float>(acc[i][j][4 * q + 2]) * lsv[i];
-              float v3 = static_cast<float>(acc[i][j][4 * q + 3]) * lsv[i];
-              if constexpr (HAS_RS) {
-                v0 = v0 * rs4.x; v1 = v1 * rs4.y; v2 = v2 * rs4.z; v3 = v3 * rs4.w;
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                const int nl = brow0 + 32 * j + 8 * q + 4 * h;
+                float4 rs4 = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+                if constexpr (HAS_RS) rs4 = *reinterpret_cast<const float4*>(sc + 1024 + nl * 4);
+                float v0 = static_cast<float>(acc[i][j][4 * q]) * lsv[i];
+                float v1 = static_cast<float>(acc[i][j][4 * q + 1]) * lsv[i];
+                float v2 = static_cast<float>(acc[i][j][4 * q + 2]) * lsv[i];
+                float v3 = static_cast<float>(acc[i][j][4 * q + 3]) * lsv[i];
+                if constexpr (HAS_RS) {
+                  v0 = v0 * rs4.x; v1 = v1 * rs4.y; v2 = v2 * rs4.z; v3 = v3 * rs4.w;
+                }
+                *reinterpret_cast<uint2*>(stg + (32 * ii + r32) * kEPitch + nl * 2) =
+                    make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+                acc[i][j][4 * q] = 0; acc[i][j][4 * q + 1] = 0; acc[i][j][4 * q + 2] = 0; acc[i][j][4 * q + 3] = 0;
               }
-              *reinterpret_cast<uint2*>(stg + r32 * kEPitch + nl * 2) =
-                  make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
-              acc[i][j][4 * q] = 0; acc[i][j][4 * q + 1] = 0; acc[i][j][4 * q + 2] = 0; acc[i][j][4 * q + 3] = 0;
-            }
           }
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
         asm volatile("s_barrier" ::: "memory");
 #pragma unroll
-        for (int it = 0; it < kERows * 32 / THR; ++it) {
+        for (int it = 0; it < 2048 / THR; ++it) {
           const int c = tid + THR * it, row = c >> 5, seg = c & 31;
           const uint8_t* src = stg + row * kEPitch + 16 * seg;
           const uint2 lo = *reinterpret_cast<const uint2*>(src);
           const uint2 hi = *reinterpret_cast<const uint2*>(src + 8);
-          const int ml = kERows * round + row;
+          const int ml = 64 * round + row;
           const bool in = n0 + 8 * seg < g.N;
           if constexpr (CDT == RK_BF16) {
             const uint32_t off = in ? static_cast<uint32_t>((ml * g.ldc + 8 * seg) * 2) : 0x80000000u;
@@ -972,7 +946,7 @@ static int gemm_kernel_override() {
 }
 
 // The persistent kernel needs K % 64 == 0 and at least 4 k-steps (the scale buffers of two
-// tiles are reused every other tile, refilled S - 1 = 3 steps ahead), and output offsets
+// tiles are reused every other tile, refilled S - 1 = 2 steps ahead), and output offsets
 // well inside 32 bits (stores of columns past N go to an offset past the descriptor).
 static bool pipe_supported(const GemmArgs& g, int es) {
   return g.K >= 256 && g.M > 16 && 256 * g.ldc * es <= (int64_t{1} << 30) &&
