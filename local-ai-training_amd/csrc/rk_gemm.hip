@@ -924,11 +924,15 @@ static void launch_gemv(const GemmArgs& g, hipStream_t stream) {
   int8_gemv_kernel<KIND, CDT, HAS_RS><<<dim3(static_cast<unsigned>(blocks)), 256, 0, stream>>>(g);
 }
 
-// 256 x 256 tiles for K >= 1024 when they still give every CU a tile, 128 x 128
-// otherwise.
+// 256 x 256 tiles for K >= 1024 when they give about 70% of the CUs a tile, 128 x 128
+// otherwise (us, small / large: 7000 x 2048 x 2048, 224 large tiles, 44.6 / 36.8; 6000 x 2048 x
+// 4096, 192 tiles, 69.8 / 60.6; 2500 x 5632 x 2048, 220 tiles, 48.6 / 38.9; 3500 x 3072 x 2048,
+// 168 tiles, 35.0 / 34.4).
+constexpr int64_t kLargeTiles = 176;
+
 static bool use_big_tiles(const GemmArgs& g) {
   const int64_t big = ((g.M + 255) / 256) * ((g.N + 255) / 256);
-  return g.K >= 1024 && big >= 256;
+  return g.K >= 1024 && big >= kLargeTiles;
 }
 
 // Kernel choice for aligned token-sized GEMMs: RATCHET_GEMM_KERNEL=ring forces the
@@ -962,7 +966,7 @@ static bool use_pipe(const GemmArgs& g, int es) {
   const int mode = gemm_kernel_override();
   if (mode != 0) return mode == 2;
   const int64_t tiles = ((g.M + kPipeBM - 1) / kPipeBM) * ((g.N + kPipeBN - 1) / kPipeBN);
-  return g.N >= 4096 && tiles >= 256;
+  return g.N >= 4096 && tiles >= kLargeTiles;
 }
 
 template <int KIND, int CDT, bool HAS_RS, bool TAIL>
@@ -978,20 +982,69 @@ static void launch_pipe(const GemmArgs& g, hipStream_t stream) {
 }
 
 template <int KIND, int CDT, bool HAS_RS, bool TAIL>
-static void launch_tiles(const GemmArgs& g, hipStream_t stream) {
-  if (use_pipe(g, CDT == RK_BF16 ? 2 : 4)) {
+static void launch_large(const GemmArgs& g, bool pipe, hipStream_t stream) {
+  if (pipe) {
     launch_pipe<KIND, CDT, HAS_RS, TAIL>(g, stream);
     return;
   }
-  if (use_big_tiles(g)) {
-    const int64_t tiles = ((g.M + 255) / 256) * ((g.N + 255) / 256);
-    int8_gemm_m32_kernel<KIND, CDT, HAS_RS, CfgBig, TAIL>
-        <<<dim3(static_cast<unsigned>(tiles)), CfgBig::THREADS, 0, stream>>>(g);
-  } else {
-    const int64_t tiles = ((g.M + 127) / 128) * ((g.N + 127) / 128);
-    int8_gemm_m32_kernel<KIND, CDT, HAS_RS, CfgSmall, TAIL>
-        <<<dim3(static_cast<unsigned>(tiles)), CfgSmall::THREADS, 0, stream>>>(g);
+  const int64_t tiles = ((g.M + 255) / 256) * ((g.N + 255) / 256);
+  int8_gemm_m32_kernel<KIND, CDT, HAS_RS, CfgBig, TAIL>
+      <<<dim3(static_cast<unsigned>(tiles)), CfgBig::THREADS, 0, stream>>>(g);
+}
+
+template <int KIND, int CDT, bool HAS_RS, bool TAIL>
+static void launch_small(const GemmArgs& g, hipStream_t stream) {
+  const int64_t tiles = ((g.M + 127) / 128) * ((g.N + 127) / 128);
+  int8_gemm_m32_kernel<KIND, CDT, HAS_RS, CfgSmall, TAIL>
+      <<<dim3(static_cast<unsigned>(tiles)), CfgSmall::THREADS, 0, stream>>>(g);
+}
+
+// Rows [0, result) of an output that takes 256 x 256 tiles go to whole rounds of them (one per
+// CU), the rest to 128 x 128 tiles in a second launch; 0: everything in one launch. In units of
+// a full round, a launch of small tiles costs about 0.5 while each has a CU to itself and 0.7
+// for a full round of two per CU. Run back to back for 0.15 s each (us, one launch / two):
+// 3108 x 6144 x 2048 71.4 / 55.4, 5003 x 4096 x 2048 71.6 / 56.8, 9000 x 2048 x 2048 67.8 /
+// 54.1, grad_input 8900 x 2304 x 3392 102.7 / 84.1, 7000 x 5632 x 2048 108.4 / 101.
+static int64_t large_tile_rows(int64_t M, int64_t N) {
+  const int64_t tiles_n = (N + 255) / 256, tiles = ((M + 255) / 256) * tiles_n;
+  int64_t best_rows = 0;
+  double best = static_cast<double>((tiles + 255) / 256);
+  for (int64_t r = tiles / 256; r >= 1; --r) {
+    const int64_t panels = r * 256 / tiles_n, rows = panels * 256;
+    if (panels == 0 || rows >= M) continue;
+    const int64_t small = ((M - rows + 127) / 128) * ((N + 127) / 128);
+    const double cost = static_cast<double>((panels * tiles_n + 255) / 256) +
+                        (small <= 256 ? 0.5 : 0.7 * static_cast<double>((small + 511) / 512));
+    if (cost < best) {
+      best = cost;
+      best_rows = rows;
+    }
   }
+  return best_rows;
+}
+
+template <int KIND, int CDT, bool HAS_RS, bool TAIL>
+static void launch_tiles(const GemmArgs& g, hipStream_t stream) {
+  const int es = CDT == RK_BF16 ? 2 : 4;
+  const bool pipe = use_pipe(g, es);
+  if (!pipe && !use_big_tiles(g)) {
+    launch_small<KIND, CDT, HAS_RS, TAIL>(g, stream);
+    return;
+  }
+  const int64_t rows = gemm_kernel_override() ? 0 : large_tile_rows(g.M, g.N);
+  if (rows == 0) {
+    launch_large<KIND, CDT, HAS_RS, TAIL>(g, pipe, stream);
+    return;
+  }
+  GemmArgs top = g, rest = g;
+  top.M = rows;
+  rest.M = g.M - rows;
+  rest.A = g.A + rows * g.lda;
+  rest.ls = g.ls + rows;
+  rest.C = static_cast<char*>(g.C) + rows * g.ldc * es;
+  if (g.R) rest.R = g.R + rows * g.ldr;
+  launch_large<KIND, CDT, HAS_RS, TAIL>(top, pipe, stream);
+  launch_small<KIND, CDT, HAS_RS, TAIL>(rest, stream);
 }
 
 template <int KIND, int CDT, bool HAS_RS>
