@@ -998,7 +998,9 @@ std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& grad, const 
   };
   const c10::DeviceGuard guard(q.device());
   const Tensor qq = rows(q), kk = rows(k), vv = rows(v), oo = rows(o), gg = rows(grad);
-  const auto out = [&] { return at::empty({B, S, H, D}, q.options()).permute({0, 2, 1, 3}); };
+  const auto out = [&] {
+    return at::empty_strided({B, H, S, D}, {S * H * D, D, H * D, 1}, q.options());
+  };
   Tensor dq = out(), dk = out(), dv = out();
   if (q.numel() == 0) return {dq, dk, dv};
   Tensor work = at::empty({rk_attention_backward_work(B, H, S)}, lse.options());

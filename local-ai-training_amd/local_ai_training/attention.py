@@ -70,7 +70,20 @@ def _backward_fits(tensors: tuple[Tensor, ...]) -> bool:
     b, h, s, d = tensors[0].shape
     padded = -(-s // 128) * 128
     return (d == 128 and 8 * b * h * padded < 2**31
-            and all(((padded + 64) * t.stride(2) + d) * 2 < 2**31 for t in tensors))
+            and ((padded + 64) * max(t.stride(2) for t in tensors) + d) * 2 < 2**31)
+
+
+def _attention_gradients(ctx, grad_out: Tensor) -> tuple[Tensor, Tensor, Tensor]:
+    q, k, v, out, lse = ctx.saved_tensors
+    if _backward_fits((q, k, v, out, grad_out)):
+        return ratchet().attention_backward(grad_out, q, k, v, out, lse, ctx.scale)
+    seed, offset = _philox_placeholders()
+    dq, dk, dv, _ = torch.ops.aten._scaled_dot_product_efficient_attention_backward(
+        grad_out, q, k, v, None, out, lse, seed, offset, 0.0, [True, True, True, False], True)
+    return dq, dk, dv
+
+
+_once_differentiable_gradients = once_differentiable(_attention_gradients)
 
 
 class CausalAttentionFn(torch.autograd.Function):
@@ -85,16 +98,10 @@ class CausalAttentionFn(torch.autograd.Function):
         return out
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, grad_out: Tensor):
-        q, k, v, out, lse = ctx.saved_tensors
-        if _backward_fits((q, k, v, out, grad_out)):
-            return ratchet().attention_backward(grad_out, q, k, v, out, lse, ctx.scale)
-        seed, offset = _philox_placeholders()
-        dq, dk, dv, _ = torch.ops.aten._scaled_dot_product_efficient_attention_backward(
-            grad_out, q, k, v, None, out, lse, seed, offset, 0.0,
-            [True, True, True, False], True)
-        return dq, dk, dv
+        if torch.is_grad_enabled():  # create_graph: the gradients, but no second derivative
+            return _once_differentiable_gradients(ctx, grad_out)
+        return _attention_gradients(ctx, grad_out)
 
 
 def causal_attention(q: Tensor, k: Tensor, v: Tensor) -> Tensor:

@@ -285,14 +285,15 @@ class _RatchetMatmul(torch.autograd.Function):
             grad_output = grad_outputs[0]
         packed = layer.packed
         mode = layer.matmul_mode
+        saved = ctx.saved_tensors
         if ctx.used_fused_int8:
-            q, s, scale = ctx.saved_tensors  # the saved int8 activations and their scales
+            q, s, scale = saved  # the saved int8 activations and their scales
             inputs_bf16 = None
             if not layer.fuse_backward_update:
                 inputs_bf16 = dequant_bf16(q, s)
             inputs_fp32 = None
         else:
-            flat_inputs, scale = ctx.saved_tensors
+            flat_inputs, scale = saved
             inputs_bf16 = None  # bf16(inputs), made only where a path needs the copy
             inputs_fp32 = flat_inputs.to(torch.float32) if mode == "fp32" else None
         # grad_weight on a side stream next to the SR quant and grad_input (below)
@@ -376,7 +377,7 @@ class _RatchetMatmul(torch.autograd.Function):
                 main.wait_stream(side)
                 side = None
             else:
-                for t in (g_w, *ctx.saved_tensors):
+                for t in (g_w, *saved):
                     t.record_stream(side)
 
         if mode == "fp32":
@@ -389,7 +390,7 @@ class _RatchetMatmul(torch.autograd.Function):
             if g.dtype not in (torch.float32, torch.bfloat16):
                 g = g.float()
             if partials is None and g.dtype == torch.float32 \
-                    and _grad_weight_supported(g, ctx.saved_tensors[0]):
+                    and _grad_weight_supported(g, q):
                 # The same pass writes bf16(g), the grad_weight GEMM's gradient operand
                 # (grad_out_tile.to(bf16), ratchet.py:162), so that GEMM reads 2-byte
                 # values instead of converting float32 ones.
@@ -670,6 +671,21 @@ def _side_stream(device: torch.device) -> torch.cuda.Stream:
 # ---------------------------------------------------------------------------
 class DiscreteRatchetLinear(nn.Module):
     """Linear layer with integer codes and pressure, but no master weight parameter."""
+
+    # per-step state: plain attributes, never parameters, buffers or modules, so setting them
+    # skips nn.Module's registration checks (13 settings per training step of a layer, a
+    # microsecond each; eager steps of small layers are bound by host work)
+    _PLAIN_ATTRIBUTES = frozenset((
+        "_pending_stats_total_weights", "_pending_counts", "_pending_rms_means", "_nonfinite",
+        "_rms_slot_mean", "_counts_snapshot", "_slot_dirty", "_queued", "_generation",
+        "_gw_workspace", "_last_rms_mean", "last_weight_gradient", "last_sr_seed",
+    ))
+
+    def __setattr__(self, name: str, value) -> None:
+        if name in self._PLAIN_ATTRIBUTES:
+            object.__setattr__(self, name, value)
+        else:
+            super().__setattr__(name, value)
 
     # fused backward under HIP-graph capture: grad_weight on a side stream, concurrent with
     # grad_input (False: one stream, e.g. to compare the two)
@@ -1117,7 +1133,7 @@ class DiscreteRatchetLinear(nn.Module):
                     own = snap if snap is not None else counts.clone()
                 else:
                     own = counts
-                pos, neg, bpos, bneg = own[0], own[1], own[2], own[3]
+                pos, neg, bpos, bneg = own.unbind()
             stats = RatchetUpdateStats(
                 total_weights=self._pending_stats_total_weights,
                 positive_moves=pos,
