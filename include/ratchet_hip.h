@@ -679,6 +679,19 @@ int rk_attention_backward(const uint16_t* q, int64_t sqb, int64_t sqh, int64_t s
                           float scale, uint16_t* dq, uint16_t* dk, uint16_t* dv, int64_t sxb,
                           int64_t sxh, int64_t sxs, float* work, void* stream);
 
+/*
+ * Appends a prompt's keys and values to a cache: k and v [B, H, S, D] (element strides; unit
+ * feature stride) go to positions start .. start + S - 1 of keys and values (one contiguous
+ * [B, H, max_len, D] buffer each, the same element size, 2 or 4 bytes), and positions
+ * start + S .. clear_to - 1 are zeroed (none when clear_to <= start + S). Rows of D elements are
+ * whole 16-byte vectors, all rows 16-byte aligned; otherwise RK_ERR_UNSUPPORTED.
+ * No counterpart in the reference (its window is recomputed per token, generate.py:183-201).
+ */
+int rk_kv_append(const void* k, int64_t skb, int64_t skh, int64_t sks, const void* v,
+                 int64_t svb, int64_t svh, int64_t svs, void* keys, void* values, int elem_size,
+                 int64_t B, int64_t H, int64_t S, int64_t D, int64_t max_len, int64_t start,
+                 int64_t clear_to, void* stream);
+
 /* HBM streaming probe (measurement only; no counterpart in the reference): reads `bytes`
  * (a multiple of 16) from src in 16-byte vectors, `unroll` (1, 2, 4, 8) loads in flight
  * per thread, `blocks` blocks of 256 threads in a grid-stride loop; copy != 0 writes them

@@ -1017,6 +1017,30 @@ std::tuple<Tensor, Tensor, Tensor> attention_backward(const Tensor& grad, const 
   return {dq, dk, dv};
 }
 
+// A prompt's k, v [B, H, S, D] into the cache buffers at `start`, the positions behind them up to
+// `clear_to` zeroed (rk_kv_append).
+void kv_append(const Tensor& k, const Tensor& v, Tensor& keys, Tensor& values, int64_t start,
+               int64_t clear_to) {
+  require_gpu(k, "kv append");
+  for (const Tensor* t : {&v, static_cast<const Tensor*>(&keys), static_cast<const Tensor*>(&values)}) {
+    same_device(k, *t, "kv append");
+    TORCH_CHECK(t->scalar_type() == k.scalar_type(), "kv append: one dtype");
+  }
+  TORCH_CHECK(k.dim() == 4 && v.sizes() == k.sizes() && k.stride(3) == 1 && v.stride(3) == 1,
+              "kv append: k and v must share a [B, H, S, D] shape with unit feature stride");
+  TORCH_CHECK(keys.dim() == 4 && values.sizes() == keys.sizes() && keys.is_contiguous() &&
+                  values.is_contiguous() && keys.size(0) == k.size(0) &&
+                  keys.size(1) == k.size(1) && keys.size(3) == k.size(3),
+              "kv append: keys and values must be contiguous [B, H, max_len, D] buffers");
+  const c10::DeviceGuard guard(k.device());
+  check_status(rk_kv_append(k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(),
+                            v.stride(0), v.stride(1), v.stride(2), keys.data_ptr(),
+                            values.data_ptr(), static_cast<int>(k.element_size()), k.size(0),
+                            k.size(1), k.size(2), k.size(3), keys.size(2), start, clear_to,
+                            stream_of(k)),
+               "rk_kv_append");
+}
+
 // Means of segments [offsets[s], offsets[s + 1]) of a float32 row-rms buffer (rk_row_rms_means).
 Tensor row_rms_means(const Tensor& row_rms, const Tensor& offsets) {
   require_gpu(row_rms, "row rms means");
@@ -1166,6 +1190,8 @@ TORCH_LIBRARY(ratchet, m) {
   m.def("attention_forward(Tensor q, Tensor k, Tensor v, float scale) -> (Tensor, Tensor)");
   m.def("attention_backward(Tensor grad, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, "
         "float scale) -> (Tensor, Tensor, Tensor)");
+  m.def("kv_append(Tensor k, Tensor v, Tensor(a!) keys, Tensor(b!) values, int start, "
+        "int clear_to) -> ()");
   m.def("cross_entropy_forward(Tensor logits, Tensor targets, int ignore_index=-100) -> "
         "(Tensor, Tensor, Tensor)");
   m.def("cross_entropy_backward(Tensor grad_loss, Tensor logits, Tensor targets, Tensor stats, "
@@ -1208,6 +1234,7 @@ TORCH_LIBRARY_IMPL(ratchet, CUDA, m) {
   m.impl("row_rms_means", &row_rms_means);
   m.impl("attention_forward", &attention_forward);
   m.impl("attention_backward", &attention_backward);
+  m.impl("kv_append", &kv_append);
   m.impl("cross_entropy_forward", &cross_entropy_forward);
   m.impl("cross_entropy_backward", &cross_entropy_backward);
 }

@@ -162,9 +162,62 @@ void attn_fwd_kernel(AttnArgs a) {
   }
 }
 
+// Keys and values of a prompt into their cache, one 16-byte vector of each per thread, the rows
+// behind them cleared in the same pass: two strided copies and two strided clears before (29 us
+// a layer at 4 sequences x 777 positions x 16 heads x 128; 10.4 us in one launch).
+__global__ __launch_bounds__(256) void kv_append_kernel(
+    const uint4* k, int64_t skb, int64_t skh, int64_t sks, const uint4* v, int64_t svb,
+    int64_t svh, int64_t svs, uint4* keys, uint4* values, uint32_t H, uint32_t S, uint32_t rows,
+    uint32_t per_row, uint32_t max_len, uint32_t start) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;  // the host bounds rows * per_row
+  const uint32_t row = i / per_row, piece = i - row * per_row;
+  if (row >= rows) return;
+  const uint32_t bh = blockIdx.y, b = bh / H, h = bh - b * H;
+  uint4 kv = make_uint4(0, 0, 0, 0), vv = kv;
+  if (row < S) {
+    kv = k[b * skb + h * skh + row * sks + piece];
+    vv = v[b * svb + h * svh + row * svs + piece];
+  }
+  const int64_t to = (static_cast<int64_t>(bh) * max_len + start + row) * per_row + piece;
+  keys[to] = kv;
+  values[to] = vv;
+}
+
 }  // namespace rk
 
 using namespace rk;
+
+extern "C" int rk_kv_append(const void* k, int64_t skb, int64_t skh, int64_t sks, const void* v,
+                            int64_t svb, int64_t svh, int64_t svs, void* keys, void* values,
+                            int elem_size, int64_t B, int64_t H, int64_t S, int64_t D,
+                            int64_t max_len, int64_t start, int64_t clear_to, void* stream) {
+  clear_error();
+  if (B < 0 || H < 0 || S < 0 || D <= 0) return fail(RK_ERR_ARG, "invalid cache shape");
+  if (start < 0 || start + S > max_len || clear_to > max_len)
+    return fail(RK_ERR_ARG, "positions past the cache");
+  if (elem_size != 2 && elem_size != 4) return fail(RK_ERR_UNSUPPORTED, "2 or 4 byte elements");
+  const int64_t end = clear_to > start + S ? clear_to : start + S;
+  if (B == 0 || H == 0 || end == start) return RK_OK;
+  if (!keys || !values || (S > 0 && (!k || !v))) return fail(RK_ERR_ARG, "null pointer");
+  const int64_t per = 16 / elem_size;  // elements per vector
+  const int64_t strides[] = {skb, skh, sks, svb, svh, svs, D};
+  for (int64_t st : strides)
+    if (st < 0 || st % per != 0)
+      return fail(RK_ERR_UNSUPPORTED, "cache rows and strides must be whole 16-byte vectors");
+  if (!aligned16(k) || !aligned16(v) || !aligned16(keys) || !aligned16(values))
+    return fail(RK_ERR_UNSUPPORTED, "keys and values need 16-byte alignment");
+  const int64_t rows = end - start, pieces = rows * (D / per);
+  if (B * H > 65535 || pieces >= (int64_t{1} << 31) || max_len >= (int64_t{1} << 31))
+    return fail(RK_ERR_UNSUPPORTED, "cache too large for one launch");
+  const dim3 grid(static_cast<unsigned>((pieces + 255) / 256), static_cast<unsigned>(B * H));
+  kv_append_kernel<<<grid, 256, 0, as_stream(stream)>>>(
+      static_cast<const uint4*>(k), skb / per, skh / per, sks / per, static_cast<const uint4*>(v),
+      svb / per, svh / per, svs / per, static_cast<uint4*>(keys), static_cast<uint4*>(values),
+      static_cast<uint32_t>(H), static_cast<uint32_t>(S), static_cast<uint32_t>(rows),
+      static_cast<uint32_t>(D / per), static_cast<uint32_t>(max_len),
+      static_cast<uint32_t>(start));
+  return launch_status("kv_append");
+}
 
 extern "C" int rk_attention_forward(const uint16_t* q, int64_t sqb, int64_t sqh, int64_t sqs,
                                     const uint16_t* k, int64_t skb, int64_t skh, int64_t sks,

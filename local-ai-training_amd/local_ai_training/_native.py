@@ -126,6 +126,8 @@ SIGNATURES: dict[str, list] = {
     "rk_attention_backward_work": [_i64, _i64, _i64],
     "rk_attention_backward": [*([_p, _i64, _i64, _i64] * 5), _p, _i64, _i64, _i64, _i64, _f32,
                               _p, _p, _p, _i64, _i64, _i64, _p, _p],
+    "rk_kv_append": [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _p, _i32, _i64, _i64,
+                     _i64, _i64, _i64, _i64, _i64, _p],
     "rk_version": [],
     "rk_last_error": [],
 }

@@ -101,6 +101,21 @@ def _is_int8(layer: nn.Module) -> bool:
     return getattr(layer, "matmul_mode", "fp32") == "int8"
 
 
+def _hip_append_supported(cache, k: Tensor, v: Tensor) -> bool:
+    """Whether ``rk_kv_append`` takes this prompt: nothing differentiated, the cache's shape and
+    GPU, 2- or 4-byte elements, rows and strides of whole 16-byte vectors, 16-byte alignment."""
+    size = k.element_size()
+    shape = (cache.batch, cache.n_head, k.shape[2], cache.head_size)
+    return (k.is_cuda and not torch.is_grad_enabled() and size in (2, 4)
+            and cache.device.type == "cuda" and k.shape == v.shape == shape
+            and v.dtype == k.dtype and (cache.device.index in (None, k.device.index))
+            and cache.batch * cache.n_head <= 65535
+            and cache.max_len * cache.head_size * size < 2**31
+            and all(t.stride(3) == 1 and t.data_ptr() % 16 == 0
+                    and not any(st * size % 16 for st in (*t.stride()[:3], cache.head_size))
+                    for t in (k, v)))
+
+
 class KVCache:
     """Per-layer keys/values [B, H, max_len, D] for incremental decoding, plus the number of
     filled positions. ``pos`` is that number as a device tensor, so a decode step (which
@@ -120,18 +135,43 @@ class KVCache:
         self._mask: Tensor | None = None
         self.step_buffers: dict[str, Tensor] = {}  # fixed-shape work buffers of a step
 
-    def buffers(self, layer: int, like: Tensor, written: int = 0) -> tuple[Tensor, Tensor]:
+    def buffers(self, layer: int, like: Tensor) -> tuple[Tensor, Tensor]:
         """The layer's key/value buffers, allocated on first use in the cache dtype
         (``like``'s when none was given) and kept from then on (later steps convert to
-        their dtype, so keys written by a prefill are never dropped). New buffers are zero,
-        but for the first ``written`` positions, which the caller writes at once."""
+        their dtype, so keys written by a prefill are never dropped)."""
         if self.keys[layer] is None:
             dtype = self.dtype or like.dtype
             shape = (self.batch, self.n_head, self.max_len, self.head_size)
-            for side in (self.keys, self.values):
-                side[layer] = torch.empty(shape, dtype=dtype, device=self.device)
-                side[layer][:, :, written:].zero_()
+            self.keys[layer] = torch.zeros(shape, dtype=dtype, device=self.device)
+            self.values[layer] = torch.zeros(shape, dtype=dtype, device=self.device)
         return self.keys[layer], self.values[layer]
+
+    def append(self, layer: int, k: Tensor, v: Tensor) -> tuple[Tensor, Tensor, Tensor, Tensor]:
+        """Writes a prompt's keys and values [B, H, S, D] at positions ``length`` .. of the
+        layer's buffers; returns them in the cache's dtype, then the buffers. On the GPU one
+        launch copies both and clears the rest of new buffers; elsewhere (and where gradients
+        flow, or rows are not whole 16-byte vectors) torch's copies."""
+        start, end = self.length, self.length + k.shape[2]
+        kept = self.keys[layer]
+        dtype = (self.dtype or k.dtype) if kept is None else kept.dtype
+        if k.dtype != dtype:
+            k, v = k.to(dtype), v.to(dtype)
+        if end > self.max_len:
+            raise ValueError("KV cache is full")
+        if _hip_append_supported(self, k, v):
+            from .ops import ratchet as _ops
+
+            if kept is None:
+                shape = (self.batch, self.n_head, self.max_len, self.head_size)
+                self.keys[layer] = torch.empty(shape, dtype=dtype, device=self.device)
+                self.values[layer] = torch.empty(shape, dtype=dtype, device=self.device)
+            keys, values = self.keys[layer], self.values[layer]
+            _ops().kv_append(k, v, keys, values, start, self.max_len if kept is None else 0)
+        else:
+            keys, values = self.buffers(layer, k)
+            keys[:, :, start:end] = k
+            values[:, :, start:end] = v
+        return k, v, keys, values
 
     def stores_bf16(self, layer: int) -> bool:
         """Whether the layer's keys and values are (or will be) stored as bfloat16."""
@@ -297,23 +337,20 @@ class CausalSelfAttention(nn.Module):
         values. ``decode``: one token at the device-side position ``cache.pos``, attending
         over the whole buffer under a mask (fixed shapes); otherwise a prompt of S tokens
         written at the host-side ``cache.length`` (causal among themselves)."""
-        start, length = cache.length, q.shape[2]
-        keys, values = cache.buffers(layer, k,
-                                     length if not decode and start == 0
-                                     and length <= cache.max_len else 0)
         out_dtype = q.dtype
-        if keys.dtype != q.dtype:
-            q, k, v = q.to(keys.dtype), k.to(keys.dtype), v.to(keys.dtype)
         if decode:
+            keys, values = cache.buffers(layer, k)
+            if keys.dtype != q.dtype:
+                q, k, v = q.to(keys.dtype), k.to(keys.dtype), v.to(keys.dtype)
             keys.index_copy_(2, cache.pos, k)
             values.index_copy_(2, cache.pos, v)
             out = _attend(q, keys, values, attn_mask=cache.decode_mask(q.dtype))
             return out.to(out_dtype)
+        start, length = cache.length, q.shape[2]
         end = start + length
-        if end > cache.max_len:
-            raise ValueError("KV cache is full")
-        keys[:, :, start:end] = k
-        values[:, :, start:end] = v
+        k, v, keys, values = cache.append(layer, k, v)
+        if keys.dtype != q.dtype:
+            q = q.to(keys.dtype)
         if start == 0:
             return _attend(q, k, v, is_causal=True).to(out_dtype)
         mask = torch.ones(length, end, dtype=torch.bool, device=q.device).tril(diagonal=start)

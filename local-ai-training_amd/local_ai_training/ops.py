@@ -178,6 +178,10 @@ def _register_fakes() -> None:
         b, h, sl, d = q.shape
         return tuple(q.new_empty((b, sl, h, d)).permute(0, 2, 1, 3) for _ in range(3))
 
+    @fake("ratchet::kv_append")
+    def _kv_append(k, v, keys, values, start, clear_to):
+        return None
+
     @fake("ratchet::row_rms_means")
     def _row_rms_means(row_rms, offsets):
         return row_rms.new_empty((offsets.shape[0] - 1,))
@@ -194,7 +198,7 @@ def _register_fakes() -> None:
 
 
 # the operators the library defines (the opcheck tests walk this list), but for
-# attention_backward, whose opcheck is beside its own tests
+# attention_backward and kv_append, whose opchecks are beside their own tests
 OPERATORS = (
     "quantize_rows", "int8_mm_nt", "packed_mm", "packed_mm_residual", "packed_mm_accumulate",
     "packed_mm_t", "unpack_transpose", "unpack", "effective_bf16", "grad_input_bf16",

@@ -37,3 +37,55 @@ def test_prefill_equals_the_float32_hand_over(cuda, monkeypatch, cache_dtype, pr
         assert a.dtype == b.dtype and torch.equal(a, b)
     for t in cache.keys + cache.values:
         assert not t[:, :, sum(prompt):].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("batch,heads,head,length", [(3, 4, 64, 1), (2, 5, 128, 40), (1, 2, 8, 7)])
+def test_append_writes_what_torch_copies_write(cuda, monkeypatch, dtype, batch, heads, head,
+                                               length):
+    """Two prompts one after the other, strided keys and values, every position compared."""
+    import local_ai_training.model as model_mod
+
+    gen = torch.Generator(device=cuda).manual_seed(length)
+    rows = torch.randn(batch, 2 * length + 3, 3 * heads * head, generator=gen, device=cuda).to(dtype)
+
+    def run():
+        cache = KVCache(1, batch, heads, head, 2 * length + 9, cuda, dtype=dtype)
+        for first, last in ((0, length), (length, 2 * length + 3)):
+            _, k, v = (t.unflatten(-1, (heads, head)).transpose(1, 2)
+                       for t in rows[:, first:last].chunk(3, dim=-1))
+            # a fresh buffer must not show what its memory held before
+            torch.full((batch, heads, 2 * length + 9, head), 5.0, device=cuda, dtype=dtype)
+            with torch.no_grad():
+                cache.append(0, k, v)
+            cache.length = last
+        return cache.keys[0], cache.values[0]
+
+    got = run()
+    monkeypatch.setattr(model_mod, "_hip_append_supported", lambda cache, k, v: False)
+    for a, b in zip(got, run()):
+        assert torch.equal(a, b)
+
+
+def test_append_refuses_what_does_not_fit(cuda):
+    from local_ai_training.ops import ratchet
+
+    keys = torch.zeros(1, 2, 10, 64, device=cuda, dtype=torch.bfloat16)
+    k = torch.ones(1, 2, 4, 64, device=cuda, dtype=torch.bfloat16)
+    for start, clear_to in ((7, 0), (-1, 0), (0, 11)):
+        with pytest.raises(RuntimeError, match="past the cache"):
+            ratchet().kv_append(k, k, keys, keys.clone(), start, clear_to)
+    with pytest.raises(RuntimeError, match="16-byte"):
+        ratchet().kv_append(k[..., :60], k[..., :60], keys[..., :60].contiguous(),
+                            keys[..., :60].contiguous(), 0, 0)
+    with pytest.raises(ValueError, match="full"):
+        KVCache(1, 1, 2, 64, 3, cuda).append(0, k, k)
+    assert not keys.any()
+
+
+def test_append_opcheck(cuda):
+    from local_ai_training.ops import ratchet
+
+    keys = torch.randn(2, 2, 12, 64, device=cuda, dtype=torch.bfloat16)
+    k = torch.randn(2, 2, 5, 64, device=cuda, dtype=torch.bfloat16)
+    torch.library.opcheck(ratchet().kv_append, (k, k * 2, keys, keys.clone(), 3, 12))
