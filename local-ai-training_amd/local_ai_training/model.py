@@ -101,10 +101,20 @@ def _is_int8(layer: nn.Module) -> bool:
     return getattr(layer, "matmul_mode", "fp32") == "int8"
 
 
-def _hip_append_supported(cache, k: Tensor, v: Tensor) -> bool:
+def _hip_append_supported(cache, layer: int, k: Tensor, v: Tensor) -> bool:
     """Whether ``rk_kv_append`` takes this prompt: nothing differentiated, the cache's shape and
-    GPU, 2- or 4-byte elements, rows and strides of whole 16-byte vectors, 16-byte alignment."""
+    GPU, 2- or 4-byte elements, rows and strides of whole 16-byte vectors, 16-byte alignment.
+    Buffers that are there must be as the cache makes them (a caller may have set others); new
+    ones are cleared only behind the prompt, so it must be at their start."""
     size = k.element_size()
+    full = (cache.batch, cache.n_head, cache.max_len, cache.head_size)
+    kept = (cache.keys[layer], cache.values[layer])
+    if kept[0] is None:
+        if cache.length:
+            return False
+    elif not all(t.shape == full and t.dtype == k.dtype and t.device == k.device
+                 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in kept):
+        return False
     shape = (cache.batch, cache.n_head, k.shape[2], cache.head_size)
     return (k.is_cuda and not torch.is_grad_enabled() and size in (2, 4)
             and cache.device.type == "cuda" and k.shape == v.shape == shape
@@ -158,7 +168,7 @@ class KVCache:
             k, v = k.to(dtype), v.to(dtype)
         if end > self.max_len:
             raise ValueError("KV cache is full")
-        if _hip_append_supported(self, k, v):
+        if _hip_append_supported(self, layer, k, v):
             from .ops import ratchet as _ops
 
             if kept is None:
@@ -197,8 +207,7 @@ class KVCache:
         self.pos.add_(steps)
 
 
-# causal training attention: the HIP forward (rk_attention_forward) where it applies, with
-# torch's memory-efficient backward (False: torch's forward too)
+# causal training attention: the HIP kernels where they apply (attention.py; False: torch's)
 hip_attention_forward = True
 _FAST_ATTENTION = [SDPBackend.EFFICIENT_ATTENTION, SDPBackend.FLASH_ATTENTION]
 _DETERMINISTIC_ATTENTION = [SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]
@@ -218,7 +227,6 @@ def _attend(q: Tensor, k: Tensor, v: Tensor, **kwargs) -> Tensor:
         if (hip_attention_forward and not deterministic and kwargs.get("is_causal")
                 and not kwargs.get("dropout_p") and kwargs.keys() <= {"is_causal", "dropout_p"}
                 and attention_supported(q, k, v)):
-            # the HIP forward with torch's memory-efficient backward (attention.py)
             return CausalAttentionFn.apply(q, k, v)
         order = _DETERMINISTIC_ATTENTION if deterministic else _FAST_ATTENTION
         with sdpa_kernel(order, set_priority=True):

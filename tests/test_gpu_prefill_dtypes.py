@@ -62,9 +62,31 @@ def test_append_writes_what_torch_copies_write(cuda, monkeypatch, dtype, batch, 
         return cache.keys[0], cache.values[0]
 
     got = run()
-    monkeypatch.setattr(model_mod, "_hip_append_supported", lambda cache, k, v: False)
+    monkeypatch.setattr(model_mod, "_hip_append_supported",
+                        lambda cache, layer, k, v: False)
     for a, b in zip(got, run()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("buffers", ["none", "strided", "float32 values"])
+def test_append_beside_its_own_buffers(cuda, buffers):
+    """A first prompt behind position 0 leaves zeros before it; buffers that the caller set are
+    written as torch's copies write them."""
+    cache = KVCache(1, 2, 3, 64, 24, cuda, dtype=torch.bfloat16)
+    cache.length = 5
+    if buffers != "none":
+        cache.keys[0] = torch.zeros(2, 24, 3, 64, device=cuda, dtype=torch.bfloat16).transpose(1, 2)
+        cache.values[0] = torch.zeros(2, 3, 24, 64, device=cuda, dtype=torch.bfloat16)
+    if buffers == "float32 values":
+        cache.keys[0], cache.values[0] = cache.keys[0].contiguous(), cache.values[0].float()
+    k, v = torch.randn(2, 2, 3, 7, 64, device=cuda).bfloat16()
+    torch.full((4, 2, 3, 24, 64), 5.0, device=cuda, dtype=torch.bfloat16)
+    with torch.no_grad():
+        cache.append(0, k, v)
+    for got, new in ((cache.keys[0], k), (cache.values[0], v)):
+        want = torch.zeros(2, 3, 24, 64, device=cuda)
+        want[:, :, 5:12] = new.float()
+        assert torch.equal(got.float(), want)
 
 
 def test_append_refuses_what_does_not_fit(cuda):
