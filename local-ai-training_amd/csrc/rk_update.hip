@@ -99,8 +99,20 @@ __global__ __launch_bounds__(256) void row_rms_segment_means_kernel(const float*
 // Element i of a 16-byte gradient vector held as four words (4 fp32, or 8 bf16 in pairs,
 // element 2j in the low half of word j).
 
+// Wavefronts (one row each) per block of the update. Every block ends in one atomic on the four
+// counters, which reach them about 17 ns apart whatever their XCD: with four rows per block a
+// layer of 6144 rows waited for its 1536 atomics. Eight (us, four / eight): 6144 x 2048 from the
+// bf16 gradient 26.5 / 18.4, 8192 x 2048 31.6 / 21.3, 3000 x 1024 13.6 / 9.7; from four splits
+// 8192 x 512 32.3 / 20.3, 2048 x 512 11.1 / 9.1. Sixteen is faster up to 4096 rows (2048 x 512
+// 8.3) and slower at 6144 (20.0) and 512 (6.3 against 5.3). The forms with more than 128
+// registers keep four: three blocks of four fit a CU's registers but one of eight (6000 x 2048
+// from two splits 32.0 / 32.9).
+template <int DT, int NC, bool ONE_SPLIT>
+constexpr int kUpdateWaves = NC >= 8 || (DT == SRC_SPLITS && NC > 1 && !ONE_SPLIT) ? 4 : 8;
+
 template <int DT, int NC, bool ZONLY, bool ONE_SPLIT = false>
-__global__ __launch_bounds__(256) void ratchet_update_grad_kernel(GradUpdateArgs a) {
+__global__ __launch_bounds__((64 * kUpdateWaves<DT, NC, ONE_SPLIT>))
+void ratchet_update_grad_kernel(GradUpdateArgs a) {
   MoveCounts cnt;
   // K opaque per row: the compiler would otherwise hoist every chunk's per-element tail
   // tests out of the row loop and hold them in registers for the whole kernel
@@ -109,8 +121,9 @@ __global__ __launch_bounds__(256) void ratchet_update_grad_kernel(GradUpdateArgs
     asm volatile("" : "+s"(K));
     return K;
   };
-  for (int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6); row < a.rows;
-       row += static_cast<int64_t>(gridDim.x) * 4) {
+  constexpr int waves = kUpdateWaves<DT, NC, ONE_SPLIT>;
+  for (int64_t row = static_cast<int64_t>(blockIdx.x) * waves + (threadIdx.x >> 6); row < a.rows;
+       row += static_cast<int64_t>(gridDim.x) * waves) {
     update_row<DT, NC, ZONLY, ONE_SPLIT>(a, row, opaque_k(), cnt);
   }
   flush_counts(cnt, a.counts);
@@ -239,10 +252,10 @@ __global__ __launch_bounds__(256) void ratchet_update_multi_kernel(const rk_upda
   flush_wave_counts(cnt, a.counts);
 }
 
-static unsigned row_grid(int64_t rows) {
+static unsigned row_grid(int64_t rows, int per_block) {
   // Enough blocks to fill 256 CUs several times over; rows beyond that loop.
-  const int64_t want = (rows + 3) / 4;
-  return static_cast<unsigned>(want < 4096 ? (want > 0 ? want : 1) : 4096);
+  const int64_t want = (rows + per_block - 1) / per_block, most = 16384 / per_block;
+  return static_cast<unsigned>(want < most ? (want > 0 ? want : 1) : most);
 }
 
 static int check_update_common(const uint8_t* packed, int64_t ldp, int64_t rows, int64_t K,
@@ -256,15 +269,22 @@ static int check_update_common(const uint8_t* packed, int64_t ldp, int64_t rows,
   return RK_OK;
 }
 
+template <int DT, int NC, bool ZONLY, bool ONE_SPLIT>
+static void launch_rows_form(const GradUpdateArgs& a, hipStream_t s) {
+  constexpr int waves = kUpdateWaves<DT, NC, ONE_SPLIT>;
+  ratchet_update_grad_kernel<DT, NC, ZONLY, ONE_SPLIT>
+      <<<row_grid(a.rows, waves), 64 * waves, 0, s>>>(a);
+}
+
 template <int DT, int NC, bool ZONLY>
 static void launch_rows(const GradUpdateArgs& a, hipStream_t s) {
   if constexpr (DT == SRC_SPLITS && NC > 0) {
     if (a.nsplit == 1) {
-      ratchet_update_grad_kernel<DT, NC, ZONLY, true><<<row_grid(a.rows), 256, 0, s>>>(a);
+      launch_rows_form<DT, NC, ZONLY, true>(a, s);
       return;
     }
   }
-  ratchet_update_grad_kernel<DT, NC, ZONLY><<<row_grid(a.rows), 256, 0, s>>>(a);
+  launch_rows_form<DT, NC, ZONLY, false>(a, s);
 }
 
 template <bool ZONLY>
@@ -404,7 +424,7 @@ extern "C" int rk_ratchet_update(uint8_t* packed, int64_t ldp, const float* z, i
   if (ldz < K) return fail(RK_ERR_ARG, "ldz < K");
   const int vec_z = aligned16(z) && (ldz % 4) == 0 && (K % 4) == 0;
   const int vec_p = (reinterpret_cast<uintptr_t>(packed) % 4) == 0 && (ldp % 4) == 0 && (K % 4) == 0;
-  ratchet_update_z_kernel<<<row_grid(rows), 256, 0, as_stream(stream)>>>(
+  ratchet_update_z_kernel<<<row_grid(rows, 4), 256, 0, as_stream(stream)>>>(
       packed, ldp, z, ldz, rows, K, max_code, threshold, low, high, counts, vec_z, vec_p);
   return launch_status("ratchet_update");
 }
