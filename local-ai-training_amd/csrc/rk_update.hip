@@ -134,19 +134,17 @@ void ratchet_update_grad_kernel(GradUpdateArgs a) {
 // space; wavefront w takes the contiguous rows [w R, (w + 1) R) and walks the layer table
 // forward as it crosses layer boundaries, each row through update_row with that layer's
 // arguments (the same code as the per-layer kernel, so the same results). Move counts add
-// up per wavefront and go to a layer's counters, four 64-bit atomics, when the wavefront
-// leaves the layer.
+// up per wavefront and go to a layer's counters, one 64-bit atomic of four lanes, when the
+// wavefront leaves the layer (four atomics one after the other: the 25M model's rows of 512
+// 157 us against 136, of 2048 39 against 34; adding a block's wavefronts up first gave no more).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void flush_wave_counts(MoveCounts& cnt, int64_t* counts) {
   const int p = wave_sum_int(cnt.pos), n = wave_sum_int(cnt.neg);
   const int bp = wave_sum_int(cnt.bpos), bn = wave_sum_int(cnt.bneg);
-  if ((threadIdx.x & 63) == 0 && counts) {
-    unsigned long long* c = reinterpret_cast<unsigned long long*>(counts);
-    if (p) atomicAdd(c + 0, static_cast<unsigned long long>(p));
-    if (n) atomicAdd(c + 1, static_cast<unsigned long long>(n));
-    if (bp) atomicAdd(c + 2, static_cast<unsigned long long>(bp));
-    if (bn) atomicAdd(c + 3, static_cast<unsigned long long>(bn));
-  }
+  const int lane = threadIdx.x & 63, v = lane == 0 ? p : lane == 1 ? n : lane == 2 ? bp : bn;
+  if (lane < 4 && counts && v)
+    atomicAdd(reinterpret_cast<unsigned long long*>(counts) + lane,
+              static_cast<unsigned long long>(v));
   cnt = MoveCounts{};
 }
 
