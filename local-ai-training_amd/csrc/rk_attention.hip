@@ -23,7 +23,7 @@
 //
 // Staging V transposed through registers (16 VALU permutes and 8-byte LDS writes per piece) and
 // its conflicts held the kernel at 36.7 us (B 32, H 8, S 512, D 64) and 112 us (B 8, H 16,
-// S 1024, D 128); both tiles by DMA and V read transposed take 21.2 and 54 us. What is left is
+// S 1024, D 128); both tiles by DMA and V read transposed take 21.2 and 59 us. What is left is
 // about the wavefront's exponentials (7 issue slots per score, as much as its MFMAs at D 128,
 // twice them at D 64) and the operands it reads (26 us for 134 MB at 5.2 TB/s).
 #include "rk_attention.h"
@@ -56,12 +56,16 @@ __device__ __forceinline__ float half_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// R keys per step: 64. At D = 128, 32 keys per step took 59 us against 54.
-template <int D, int R>
+// R keys are staged per step, U of them make one update of the running max and sum. The U keys'
+// probabilities are rounded to bf16 relative to the max after them, so U is part of the result's
+// rounding, which int8 rows downstream turn into differences of 1%: 64 at D = 64, 32 at D = 128.
+// With 64 at D = 128 too, B 8, H 16, S 1024 took 55-59 us against 59-61, B 2, H 8, S 2048 48
+// against 52.
+template <int D, int R, int U>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4)))
 void attn_fwd_kernel(AttnArgs a) {
   using T = AttnTile<D, R>;
-  constexpr int KT = R / 32;
+  constexpr int UT = U / 32;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kAttnStages * 2 * T::BYTES];
   const uint32_t lds0 = lds_address(smem);
   // positions fit 32 bits (checked by the host, with the row offsets of S + 128 rows)
@@ -95,65 +99,77 @@ void attn_fwd_kernel(AttnArgs a) {
   for (int step = 0; step < steps; ++step) {
     dma_wait_barrier<0>();
     if (step + 1 < steps) issue(step + 1);
-    const int key0 = step * R;
-    if (key0 > qw0 + 31) continue;  // above this wavefront's diagonal
     const uint8_t* kt = smem + (step % kAttnStages) * 2 * T::BYTES;
     const uint8_t* vt = kt + T::BYTES;
-    // S^T: lane holds keys key0 + 32 t + 8 (e / 4) + 4 h + e % 4 of its query
-    v16f_a st[KT];
+    if (step * R > qw0 + 31) continue;  // above this wavefront's diagonal
+    // S^T: lane holds keys step R + 32 t + 8 (e / 4) + 4 h + e % 4 of its query
+    v16f_a sc[R / 32];
 #pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      st[t] = v16f_a{};
+    for (int t = 0; t < R / 32; ++t) {
+      sc[t] = v16f_a{};
 #pragma unroll
       for (int s = 0; s < D / 16; ++s)
-        st[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(kt, 32 * t, s, lane), qf[s],
-                                                        st[t], 0, 0, 0);
+        sc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(kt, 32 * t, s, lane), qf[s],
+                                                        sc[t], 0, 0, 0);
     }
-    if (key0 + R - 1 > qw0) {  // some key of the step lies past some query
+    if (step * R + R - 1 > qw0) {  // some key of the step lies past some query
 #pragma unroll
-      for (int t = 0; t < KT; ++t)
+      for (int t = 0; t < R / 32; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-          if (key0 + 32 * t + 8 * (e / 4) + 4 * h + (e % 4) > qi) st[t][e] = -INFINITY;
+          if (step * R + 32 * t + 8 * (e / 4) + 4 * h + (e % 4) > qi) sc[t][e] = -INFINITY;
     }
-    float mx = -INFINITY;
+    // The updates' probabilities first, then their products: the only branches (a rescale) then
+    // lie between products, and the exponentials of one update overlap the next one's.
+    float alpha[R / U], ps[R / U];
+    uint4 pf[R / 32][2];
 #pragma unroll
-    for (int t = 0; t < KT; ++t)
+    for (int u = 0; u < R / U; ++u) {
+      float mx = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, st[t][e]);
-    mx = half_max(mx);
-    // the running max in base-2 units (scale * log2 e > 0 commutes with max)
-    const float mnew = fmaxf(m, mx * a.scale_log2);
-    const float mref = mnew == -INFINITY ? 0.0f : mnew;  // a row with no key yet
-    const float alpha = __builtin_amdgcn_exp2f(m - mref);
-    m = mnew;
-    // rescale only when some query's running max grew (alpha == 1 exactly otherwise:
-    // exp2(0) = 1), which after the first steps is rare
-    if (__any(alpha != 1.0f)) {
+      for (int t = u * UT; t < (u + 1) * UT; ++t)
 #pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt)
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[t][e]);
+      mx = half_max(mx);
+      // the running max in base-2 units (scale * log2 e > 0 commutes with max)
+      const float mnew = fmaxf(m, mx * a.scale_log2);
+      const float mref = mnew == -INFINITY ? 0.0f : mnew;  // a row with no key yet
+      alpha[u] = __builtin_amdgcn_exp2f(m - mref);
+      m = mnew;
+      ps[u] = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) o[dt][e] = o[dt][e] * alpha;
-    }
-    float ps = 0.0f;
+      for (int t = u * UT; t < (u + 1) * UT; ++t) {
+        float p[16];
 #pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      float p[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[t][e], a.scale_log2, -mref));
-        ps = ps + p[e];
+        for (int e = 0; e < 16; ++e) {
+          p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[t][e], a.scale_log2, -mref));
+          ps[u] = ps[u] + p[e];
+        }
+        pack16(pf[t], p);
       }
-      uint4 pf[2];
-      pack16(pf, p);
+    }
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
+    for (int u = 0; u < R / U; ++u) {
+      // keys above the diagonal: alpha is 1 and every p zero, but their values may not be finite
+      if (step * R + u * U > qw0 + 31) break;
+      // rescale only when some query's running max grew (alpha == 1 exactly otherwise:
+      // exp2(0) = 1), which after the first keys is rare
+      if (__any(alpha[u] != 1.0f)) {
 #pragma unroll
         for (int dt = 0; dt < D / 32; ++dt)
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              col_frag<D>(vt, 32 * t + 16 * s2, dt, lane), frag_of(pf[s2]), o[dt], 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o[dt][e] = o[dt][e] * alpha[u];
+      }
+      l = l * alpha[u] + half_sum(ps[u]);
+#pragma unroll
+      for (int t = u * UT; t < (u + 1) * UT; ++t)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt)
+            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                col_frag<D>(vt, 32 * t + 16 * s2, dt, lane), frag_of(pf[t][s2]), o[dt], 0, 0, 0);
     }
-    l = l * alpha + half_sum(ps);
   }
 
   if (qi < S) {
@@ -249,7 +265,7 @@ extern "C" int rk_attention_forward(const uint16_t* q, int64_t sqb, int64_t sqh,
   AttnArgs a{q, k, v, sqb, sqh, sqs, skb, skh, sks, svb, svh, svs, o, sob, soh, sos, lse,
              B, H, S, scale * 1.4426950408889634f};
   const dim3 grid(static_cast<unsigned>(blocks));
-  if (D == 64) attn_fwd_kernel<64, 64><<<grid, 256, 0, as_stream(stream)>>>(a);
-  else attn_fwd_kernel<128, 64><<<grid, 256, 0, as_stream(stream)>>>(a);
+  if (D == 64) attn_fwd_kernel<64, 64, 64><<<grid, 256, 0, as_stream(stream)>>>(a);
+  else attn_fwd_kernel<128, 64, 32><<<grid, 256, 0, as_stream(stream)>>>(a);
   return launch_status("attention_forward");
 }
