@@ -170,6 +170,13 @@ int rk_int8_gemm_packed_t(const int8_t* A, int64_t lda, const uint8_t* packed, i
                           void* stream);
 
 /*
+ * Of the M rows of an int8 GEMM with a contiguous bfloat16 output [M, N] and aligned operands, how
+ * many are computed in 256 x 256 tiles (0, whole rounds of them, or M); the rest take 128 x 128
+ * tiles. packed_t: the rk_int8_gemm_packed_t form. No device work; the results do not depend on it.
+ */
+int64_t rk_int8_gemm_large_rows(int64_t M, int64_t N, int64_t K, int packed_t);
+
+/*
  * Decode + transpose the packed state: codeT[k, n] = (packed[n, k] & 15) - max_code.
  *   packed [N, K] (row stride ldp) -> codeT int8 [K, N] (row stride ldt).
  * Feeds the int8 grad_input GEMM (contraction over the output features), replacing

@@ -924,15 +924,23 @@ static void launch_gemv(const GemmArgs& g, hipStream_t stream) {
   int8_gemv_kernel<KIND, CDT, HAS_RS><<<dim3(static_cast<unsigned>(blocks)), 256, 0, stream>>>(g);
 }
 
-// 256 x 256 tiles for K >= 1024 when they give about 70% of the CUs a tile, 128 x 128
-// otherwise (us, small / large: 7000 x 2048 x 2048, 224 large tiles, 44.6 / 36.8; 6000 x 2048 x
-// 4096, 192 tiles, 69.8 / 60.6; 2500 x 5632 x 2048, 220 tiles, 48.6 / 38.9; 3500 x 3072 x 2048,
-// 168 tiles, 35.0 / 34.4).
-constexpr int64_t kLargeTiles = 176;
+// 256 x 256 tiles for K >= 1024 (wide outputs through the persistent kernel: K >= 256) when there
+// is one for every CU. Fewer leave CUs idle for the whole launch. They still win where the small
+// tiles need a second round (three of them fit a CU, so 768 run at once), from K 1024 on (1280 in
+// the grad_input form), and from K 3072 on where those 768 are nearly all there. Time of small over
+// time of large tiles, whole 256-row panels x 2048 columns (x 4096 columns): 192 large or 768 small
+// tiles K 1024 0.93 (0.85), K 2048 1.00 (0.96), K 3072 1.11 (1.05); 208 or 832 tiles K 512 - (0.97),
+// K 1024 1.10 (1.02), K 2048 1.21 (1.18); 176 or 704 tiles K 1024 0.82 (0.81), K 3072 1.06 (1.03).
+static bool large_tiles_fill(const GemmArgs& g, bool packed_t) {
+  const int64_t large = ((g.M + 255) / 256) * ((g.N + 255) / 256);
+  if (large >= 256) return true;
+  const int64_t small = ((g.M + 127) / 128) * ((g.N + 127) / 128);
+  if (small > 768) return g.K >= (packed_t ? 1280 : 1024);
+  return small > 704 && g.K >= 3072;
+}
 
-static bool use_big_tiles(const GemmArgs& g) {
-  const int64_t big = ((g.M + 255) / 256) * ((g.N + 255) / 256);
-  return g.K >= 1024 && big >= kLargeTiles;
+static bool use_big_tiles(const GemmArgs& g, bool packed_t) {
+  return g.K >= 1024 && large_tiles_fill(g, packed_t);
 }
 
 // Kernel choice for aligned token-sized GEMMs: RATCHET_GEMM_KERNEL=ring forces the
@@ -949,9 +957,9 @@ static int gemm_kernel_override() {
   return mode;
 }
 
-// The persistent kernel needs K % 64 == 0 and at least 4 k-steps (the scale buffers of two
-// tiles are reused every other tile, refilled S - 1 = 2 steps ahead), and output offsets
-// well inside 32 bits (stores of columns past N go to an offset past the descriptor).
+// The persistent kernel needs at least 4 k-steps (the scale buffers of two tiles are reused every
+// other tile, refilled S - 1 = 2 steps ahead), and output offsets well inside 32 bits (stores of
+// columns past N go to an offset past the descriptor).
 static bool pipe_supported(const GemmArgs& g, int es) {
   return g.K >= 256 && g.M > 16 && 256 * g.ldc * es <= (int64_t{1} << 30) &&
          (g.R == nullptr || 256 * g.ldr * 4 <= (int64_t{1} << 30));
@@ -961,12 +969,11 @@ static bool pipe_supported(const GemmArgs& g, int es) {
 // 8192 x 512 float32: 218.7 / 183.6; 8192 x 8192 x 2048: 207.0 / 191.2; 8192 x 6144 x 2048:
 // 131.9 / 128.3), narrow ones the register ring (16384 x 2048 x 512: 34.2 / 36.9;
 // grad_input 16384 x 512 x 2048: 25.6 / 37.4).
-static bool use_pipe(const GemmArgs& g, int es) {
+static bool use_pipe(const GemmArgs& g, int es, bool packed_t) {
   if (!pipe_supported(g, es)) return false;
   const int mode = gemm_kernel_override();
   if (mode != 0) return mode == 2;
-  const int64_t tiles = ((g.M + kPipeBM - 1) / kPipeBM) * ((g.N + kPipeBN - 1) / kPipeBN);
-  return g.N >= 4096 && tiles >= kLargeTiles;
+  return g.N >= 4096 && large_tiles_fill(g, packed_t);
 }
 
 template <int KIND, int CDT, bool HAS_RS, bool TAIL>
@@ -1001,11 +1008,13 @@ static void launch_small(const GemmArgs& g, hipStream_t stream) {
 
 // Rows [0, result) of an output that takes 256 x 256 tiles go to whole rounds of them (one per
 // CU), the rest to 128 x 128 tiles in a second launch; 0: everything in one launch. In units of
-// a full round, a launch of small tiles costs about 0.5 while each has a CU to itself and 0.7
-// for a full round of two per CU. Run back to back for 0.15 s each (us, one launch / two):
-// 3108 x 6144 x 2048 71.4 / 55.4, 5003 x 4096 x 2048 71.6 / 56.8, 9000 x 2048 x 2048 67.8 /
-// 54.1, grad_input 8900 x 2304 x 3392 102.7 / 84.1, 7000 x 5632 x 2048 108.4 / 101.
-static int64_t large_tile_rows(int64_t M, int64_t N) {
+// a full round, a launch of small tiles costs about 0.5 + 80 / K while each has a CU to itself and
+// 0.7 + 160 / K for a full round of two per CU (the start of the launch and the output stores do
+// not shrink with K). Run back to back for 0.15 s each (us, one launch / two): 3108 x 6144 x 2048
+// 71.4 / 55.4, 5003 x 4096 x 2048 71.6 / 56.8, 9000 x 2048 x 2048 67.8 / 54.1, grad_input 8900 x
+// 2304 x 3392 102.7 / 84.1, 7000 x 5632 x 2048 108.4 / 101; 2900 x 6144 x 256 23.6 / 20.3;
+// 5003 x 8192 x 512 42.8 / 43.2, float32 60.1 / 62.3.
+static int64_t large_tile_rows(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles_n = (N + 255) / 256, tiles = ((M + 255) / 256) * tiles_n;
   int64_t best_rows = 0;
   double best = static_cast<double>((tiles + 255) / 256);
@@ -1014,7 +1023,8 @@ static int64_t large_tile_rows(int64_t M, int64_t N) {
     if (panels == 0 || rows >= M) continue;
     const int64_t small = ((M - rows + 127) / 128) * ((N + 127) / 128);
     const double cost = static_cast<double>((panels * tiles_n + 255) / 256) +
-                        (small <= 256 ? 0.5 : 0.7 * static_cast<double>((small + 511) / 512));
+                        (small <= 256 ? 0.5 : 0.7 * static_cast<double>((small + 511) / 512)) +
+                        (small <= 256 ? 80.0 : 160.0) / static_cast<double>(K);
     if (cost < best) {
       best = cost;
       best_rows = rows;
@@ -1023,16 +1033,23 @@ static int64_t large_tile_rows(int64_t M, int64_t N) {
   return best_rows;
 }
 
+// The rows of an output that go to large tiles: none, whole rounds of them, or all.
+static int64_t plan_large_rows(const GemmArgs& g, bool pipe, bool packed_t) {
+  if (!pipe && !use_big_tiles(g, packed_t)) return 0;
+  const int64_t rows = gemm_kernel_override() ? 0 : large_tile_rows(g.M, g.N, g.K);
+  return rows ? rows : g.M;
+}
+
 template <int KIND, int CDT, bool HAS_RS, bool TAIL>
 static void launch_tiles(const GemmArgs& g, hipStream_t stream) {
-  const int es = CDT == RK_BF16 ? 2 : 4;
-  const bool pipe = use_pipe(g, es);
-  if (!pipe && !use_big_tiles(g)) {
+  constexpr int es = CDT == RK_BF16 ? 2 : 4;
+  const bool pipe = use_pipe(g, es, KIND == B_PACKED_T);
+  const int64_t rows = plan_large_rows(g, pipe, KIND == B_PACKED_T);
+  if (rows == 0) {
     launch_small<KIND, CDT, HAS_RS, TAIL>(g, stream);
     return;
   }
-  const int64_t rows = gemm_kernel_override() ? 0 : large_tile_rows(g.M, g.N);
-  if (rows == 0) {
+  if (rows == g.M) {
     launch_large<KIND, CDT, HAS_RS, TAIL>(g, pipe, stream);
     return;
   }
@@ -1192,6 +1209,16 @@ extern "C" int rk_int8_gemm_packed(const int8_t* A, int64_t lda, const uint8_t* 
                                    int64_t K, void* stream) {
   return gemm_entry(A, lda, packed, ldp, B_PACKED, max_code, ls, rs, C, c_dtype, ldc, M, N, K,
                     stream);
+}
+
+extern "C" int64_t rk_int8_gemm_large_rows(int64_t M, int64_t N, int64_t K, int packed_t) {
+  if (M <= 16 || N <= 0 || K <= 0 || K % 16 != 0 || N % 8 != 0) return 0;
+  GemmArgs g{};
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.ldc = N;
+  return plan_large_rows(g, use_pipe(g, 2, packed_t != 0), packed_t != 0);
 }
 
 extern "C" int rk_int8_gemm_packed_residual(const int8_t* A, int64_t lda,

@@ -61,6 +61,7 @@ SIGNATURES: dict[str, list] = {
                             _p],
     "rk_int8_gemm_packed_t": [_p, _i64, _p, _i64, _i32, _p, _p, _p, _i32, _i64, _i64, _i64,
                               _i64, _p],
+    "rk_int8_gemm_large_rows": [_i64, _i64, _i64, _i32],
     "rk_int8_gemm_packed_residual": [_p, _i64, _p, _i64, _i32, _p, _p, _p, _i64, _p, _i64,
                                      _i64, _i64, _i64, _p],
     "rk_unpack_transpose": [_p, _i64, _i32, _p, _i64, _i64, _i64, _p],
@@ -136,6 +137,7 @@ SIGNATURES: dict[str, list] = {
 RESTYPES = {
     "rk_last_error": ctypes.c_char_p,
     "rk_attention_backward_work": ctypes.c_int64,
+    "rk_int8_gemm_large_rows": ctypes.c_int64,
     "rk_decode_attention_splits": ctypes.c_int64,
     "rk_grad_weight_update_counters": ctypes.c_int64,
     "rk_embedding_backward_workspace": ctypes.c_int64,
