@@ -40,7 +40,8 @@ struct AttnArgs {
   uint16_t* o;
   int64_t sob, soh, sos;
   float* lse;  // [B, H, S]
-  int64_t B, H, S;
+  int64_t bh0, BH;  // this launch's (batch, head) pairs: bh0 .. bh0 + BH - 1
+  int64_t H, S;
   float scale_log2;  // scale * log2(e)
 };
 
@@ -70,11 +71,11 @@ void attn_fwd_kernel(AttnArgs a) {
   const uint32_t lds0 = lds_address(smem);
   // positions fit 32 bits (checked by the host, with the row offsets of S + 128 rows)
   const int S = static_cast<int>(a.S);
-  const int64_t BH = a.B * a.H;
   const int nqb = (S + kAttnRows - 1) / kAttnRows;
-  const int blk = static_cast<int>(blockIdx.x / BH);  // heads fastest: one head stays on an XCD
-  const int qb = nqb - 1 - blk;                       // longest causal rows first
-  const int64_t bh = blockIdx.x - blk * BH, b = bh / a.H, hd = bh - b * a.H;
+  // heads fastest: with BH a multiple of 8, one head stays on an XCD
+  const int blk = static_cast<int>(blockIdx.x / a.BH);
+  const int qb = nqb - 1 - blk;  // longest causal rows first
+  const int64_t bh = a.bh0 + blockIdx.x - blk * a.BH, b = bh / a.H, hd = bh - b * a.H;
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qw0 = qb * kAttnRows + 32 * wave, qi = qw0 + l32;  // this lane's query
@@ -259,13 +260,16 @@ extern "C" int rk_attention_forward(const uint16_t* q, int64_t sqb, int64_t sqh,
   if ((rows * sqs + D) * 2 >= (int64_t{1} << 31) || (rows * sks + D) * 2 >= (int64_t{1} << 31) ||
       (rows * svs + D) * 2 >= (int64_t{1} << 31))
     return fail(RK_ERR_UNSUPPORTED, "sequence extent exceeds 2^31 bytes per head");
-  const int64_t blocks = B * H * ((S + kAttnRows - 1) / kAttnRows);
-  if (B * H > 0x7fffffff || blocks >= (int64_t{1} << 24))  // 2^32 threads
-    return fail(RK_ERR_ARG, "grid too large");
+  // a launch holds fewer than 2^24 blocks (2^32 threads): more heads take several
+  const int64_t nqb = (S + kAttnRows - 1) / kAttnRows, per = ((int64_t{1} << 24) - 1) / nqb;
+  if (B * H > 0x7fffffff || per == 0) return fail(RK_ERR_ARG, "grid too large");
   AttnArgs a{q, k, v, sqb, sqh, sqs, skb, skh, sks, svb, svh, svs, o, sob, soh, sos, lse,
-             B, H, S, scale * 1.4426950408889634f};
-  const dim3 grid(static_cast<unsigned>(blocks));
-  if (D == 64) attn_fwd_kernel<64, 64, 64><<<grid, 256, 0, as_stream(stream)>>>(a);
-  else attn_fwd_kernel<128, 64, 32><<<grid, 256, 0, as_stream(stream)>>>(a);
+             0, 0, H, S, scale * 1.4426950408889634f};
+  for (; a.bh0 < B * H; a.bh0 += a.BH) {
+    a.BH = B * H - a.bh0 < per ? B * H - a.bh0 : per;
+    const dim3 grid(static_cast<unsigned>(a.BH * nqb));
+    if (D == 64) attn_fwd_kernel<64, 64, 64><<<grid, 256, 0, as_stream(stream)>>>(a);
+    else attn_fwd_kernel<128, 64, 32><<<grid, 256, 0, as_stream(stream)>>>(a);
+  }
   return launch_status("attention_forward");
 }

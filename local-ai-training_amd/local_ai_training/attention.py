@@ -42,10 +42,12 @@ def _philox_placeholders() -> tuple[Tensor, Tensor]:
 
 def _extent_fits(shape: tuple[int, ...], stride: tuple[int, ...]) -> bool:
     """The kernel's 32-bit buffer offsets: one (batch, head)'s rows up to S + 128 (the last
-    key block's padding) within 2^31 bytes of bf16, and at most 2^31 - 1 (batch, head)
-    pairs (the same limits ``rk_attention_forward`` checks before launching)."""
+    key block's padding) within 2^31 bytes of bf16, at most 2^31 - 1 (batch, head) pairs, and
+    fewer than 2^24 blocks of 128 positions in a head (the same limits ``rk_attention_forward``
+    checks before launching)."""
     b, h, s, d = shape
-    return ((s + 128) * stride[2] + d) * 2 < 2**31 and b * h <= 0x7FFFFFFF
+    return (((s + 128) * stride[2] + d) * 2 < 2**31 and b * h <= 0x7FFFFFFF
+            and s <= 128 * (2**24 - 1))
 
 
 def attention_supported(q: Tensor, k: Tensor, v: Tensor) -> bool:
