@@ -390,9 +390,10 @@ class FeedForward(nn.Module):
         bf16_out = None
         if int8_contract and self.bf16_expand:
             bf16_out = _autocast_bf16(inputs)
-            # without gradients the GELU prologue reads the bf16 result too (the same values)
+            # without gradients the GELU prologue reads an int8 expansion's bf16 result too
+            # (the same values; any other layer's result is its own, and so are its arguments)
             if (bf16_out is None and inputs.is_cuda and inputs.dtype == torch.float32
-                    and not torch.is_grad_enabled()):
+                    and not torch.is_grad_enabled() and _is_int8(self.expand)):
                 bf16_out = torch.bfloat16
         kw = {"out_dtype": bf16_out} if bf16_out is not None else {}
         if inputs_int8 is not None:

@@ -111,3 +111,21 @@ def test_append_opcheck(cuda):
     keys = torch.randn(2, 2, 12, 64, device=cuda, dtype=torch.bfloat16)
     k = torch.randn(2, 2, 5, 64, device=cuda, dtype=torch.bfloat16)
     torch.library.opcheck(ratchet().kv_append, (k, k * 2, keys, keys.clone(), 3, 12))
+
+
+@pytest.mark.parametrize("expansion", ["int8", "fp32", "nn.Linear"])
+def test_feed_forward_without_gradients_takes_any_expansion(cuda, monkeypatch, expansion):
+    """The bf16 hand-over asks an int8 expansion only; another layer in its place is called
+    with its inputs alone and its float32 result goes on as it is."""
+    config = ModelConfig(vocab_size=64, block_size=16, n_layer=1, n_head=2, n_embd=128,
+                         ffn_hidden=256, matmul_mode="int8")
+    layer = build_seeded_model(config, max_code=3, seed=1).to(cuda).eval().blocks[0].feed_forward
+    if expansion == "nn.Linear":
+        layer.expand = torch.nn.Linear(128, 256, bias=False, device=cuda)
+    else:
+        layer.expand.matmul_mode = expansion
+    x = torch.randn(2, 7, 128, device=cuda, generator=torch.Generator(cuda).manual_seed(3))
+    with torch.no_grad():
+        got = layer(x)
+        monkeypatch.setattr(FeedForward, "bf16_expand", False)
+        assert got.dtype == torch.float32 and torch.equal(got, layer(x))
