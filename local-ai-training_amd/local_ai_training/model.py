@@ -116,9 +116,10 @@ def _hip_append_supported(cache, layer: int, k: Tensor, v: Tensor) -> bool:
                  and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in kept):
         return False
     shape = (cache.batch, cache.n_head, k.shape[2], cache.head_size)
+    # pos lies where the cache's device (a torch.device, a string, an index) resolved to
     return (k.is_cuda and not torch.is_grad_enabled() and size in (2, 4)
-            and cache.device.type == "cuda" and k.shape == v.shape == shape
-            and v.dtype == k.dtype and (cache.device.index in (None, k.device.index))
+            and cache.pos.device == k.device == v.device and k.shape == v.shape == shape
+            and v.dtype == k.dtype
             and cache.batch * cache.n_head <= 65535
             and cache.max_len * cache.head_size * size < 2**31
             and all(t.stride(3) == 1 and t.data_ptr() % 16 == 0
@@ -173,8 +174,8 @@ class KVCache:
 
             if kept is None:
                 shape = (self.batch, self.n_head, self.max_len, self.head_size)
-                self.keys[layer] = torch.empty(shape, dtype=dtype, device=self.device)
-                self.values[layer] = torch.empty(shape, dtype=dtype, device=self.device)
+                self.keys[layer] = torch.empty(shape, dtype=dtype, device=k.device)
+                self.values[layer] = torch.empty(shape, dtype=dtype, device=k.device)
             keys, values = self.keys[layer], self.values[layer]
             _ops().kv_append(k, v, keys, values, start, self.max_len if kept is None else 0)
         else:

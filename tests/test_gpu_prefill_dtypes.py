@@ -129,3 +129,14 @@ def test_feed_forward_without_gradients_takes_any_expansion(cuda, monkeypatch, e
         got = layer(x)
         monkeypatch.setattr(FeedForward, "bf16_expand", False)
         assert got.dtype == torch.float32 and torch.equal(got, layer(x))
+
+
+@pytest.mark.parametrize("device", ["cuda", "cuda:0", torch.device("cuda"), 0])
+def test_append_to_a_cache_on_a_device_of_any_form(cuda, device):
+    cache = KVCache(1, 2, 3, 64, 10, device, dtype=torch.bfloat16)
+    k, v = torch.randn(2, 2, 3, 7, 64, device=cuda).bfloat16()
+    with torch.no_grad():
+        cache.append(0, k, v)
+    for got, new in ((cache.keys[0], k), (cache.values[0], v)):
+        assert got.device == k.device and torch.equal(got[:, :, :7], new)
+        assert not got[:, :, 7:].any()
