@@ -101,17 +101,22 @@ __global__ __launch_bounds__(256) void row_rms_segment_means_kernel(const float*
 
 // Wavefronts (one row each) per block of the update. Every block ends in one atomic on the four
 // counters, which reach them about 17 ns apart whatever their XCD: with four rows per block a
-// layer of 6144 rows waited for its 1536 atomics. Eight (us, four / eight): 6144 x 2048 from the
-// bf16 gradient 26.5 / 18.4, 8192 x 2048 31.6 / 21.3, 3000 x 1024 13.6 / 9.7; from four splits
-// 8192 x 512 32.3 / 20.3, 2048 x 512 11.1 / 9.1. Sixteen is faster up to 4096 rows (2048 x 512
-// 8.3) and slower at 6144 (20.0) and 512 (6.3 against 5.3). The forms with more than 128
-// registers keep four: three blocks of four fit a CU's registers but one of eight (6000 x 2048
-// from two splits 32.0 / 32.9).
-template <int DT, int NC, bool ONE_SPLIT>
-constexpr int kUpdateWaves = NC >= 8 || (DT == SRC_SPLITS && NC > 1 && !ONE_SPLIT) ? 4 : 8;
+// layer of 6144 rows waited for its 1536 atomics. Eight from the rows given here on (us, four /
+// eight): 6144 x 2048 from the bf16 gradient 26.5 / 18.4, 8192 x 2048 31.6 / 21.3, 3000 x 1024
+// 13.6 / 9.7; from four splits 8192 x 512 32.3 / 20.3, 2048 x 512 11.1 / 9.1. Fewer rows wait for
+// their own latency, which eight wavefronts on a CU lengthen: 768 x 2048 7.0 / 7.0, 256 x 2048
+// 5.4 / 6.3, 128 x 512 5.0 / 5.4. Streamed rows (NC 0) 2048 x 8192 bf16 28.2 / 25.8, 512 x 4096
+// float32 19.8 / 22.4, 64 x 8192 14.8 / 16.8. Sixteen is faster up to 4096 rows (2048 x 512 8.3)
+// and slower at 6144 (20.0).
+// The forms with more than 128 registers keep four: three blocks of four fit a CU's registers but
+// one of eight (6000 x 2048 from two splits 32.0 / 32.9, streamed 2048 x 8192 from three 72.6 /
+// 76.2). So does the normalization alone, which has no counters (1000 x 2048 7.9 / 10.2).
+template <int DT, int NC, bool ZONLY, bool ONE_SPLIT>
+constexpr int64_t kRowsOfEight =  // 0: always four
+    ZONLY || NC >= 8 || (DT == SRC_SPLITS && NC != 1 && !ONE_SPLIT) ? 0 : (NC == 0 ? 2048 : 768);
 
-template <int DT, int NC, bool ZONLY, bool ONE_SPLIT = false>
-__global__ __launch_bounds__((64 * kUpdateWaves<DT, NC, ONE_SPLIT>))
+template <int DT, int NC, bool ZONLY, bool ONE_SPLIT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES)
 void ratchet_update_grad_kernel(GradUpdateArgs a) {
   MoveCounts cnt;
   // K opaque per row: the compiler would otherwise hoist every chunk's per-element tail
@@ -121,9 +126,8 @@ void ratchet_update_grad_kernel(GradUpdateArgs a) {
     asm volatile("" : "+s"(K));
     return K;
   };
-  constexpr int waves = kUpdateWaves<DT, NC, ONE_SPLIT>;
-  for (int64_t row = static_cast<int64_t>(blockIdx.x) * waves + (threadIdx.x >> 6); row < a.rows;
-       row += static_cast<int64_t>(gridDim.x) * waves) {
+  for (int64_t row = static_cast<int64_t>(blockIdx.x) * WAVES + (threadIdx.x >> 6); row < a.rows;
+       row += static_cast<int64_t>(gridDim.x) * WAVES) {
     update_row<DT, NC, ZONLY, ONE_SPLIT>(a, row, opaque_k(), cnt);
   }
   flush_counts(cnt, a.counts);
@@ -269,9 +273,13 @@ static int check_update_common(const uint8_t* packed, int64_t ldp, int64_t rows,
 
 template <int DT, int NC, bool ZONLY, bool ONE_SPLIT>
 static void launch_rows_form(const GradUpdateArgs& a, hipStream_t s) {
-  constexpr int waves = kUpdateWaves<DT, NC, ONE_SPLIT>;
-  ratchet_update_grad_kernel<DT, NC, ZONLY, ONE_SPLIT>
-      <<<row_grid(a.rows, waves), 64 * waves, 0, s>>>(a);
+  if constexpr (kRowsOfEight<DT, NC, ZONLY, ONE_SPLIT> > 0) {
+    if (a.rows >= kRowsOfEight<DT, NC, ZONLY, ONE_SPLIT>) {
+      ratchet_update_grad_kernel<DT, NC, ZONLY, ONE_SPLIT, 8><<<row_grid(a.rows, 8), 512, 0, s>>>(a);
+      return;
+    }
+  }
+  ratchet_update_grad_kernel<DT, NC, ZONLY, ONE_SPLIT, 4><<<row_grid(a.rows, 4), 256, 0, s>>>(a);
 }
 
 template <int DT, int NC, bool ZONLY>

@@ -1,6 +1,11 @@
-"""The update at row counts around its blocks of four and eight rows and past one row per
-wavefront of the largest grid (16384), for every source and width class, against the oracle:
-packed bytes, move counts and row rms, bit for bit.
+"""The update at row counts around its blocks of four and eight rows, around the counts that take
+blocks of eight (768, streamed rows 2048) and past one row per wavefront of the largest grid
+(16384): packed bytes, move counts and row rms, bit for bit.
+
+Every source and width class (in registers, rows of up to 512, 2048 and 6144 columns, float32 512
+and 2048; streamed beyond) is compared with the oracle at small row counts. Past 16384 rows
+the narrow classes are compared with it too; the wide ones, where it would take minutes, with
+the same rows updated in two calls, on the other side of the line or the grid.
 """
 
 from __future__ import annotations
@@ -43,3 +48,46 @@ def test_row_counts(cuda, rows, source, k):
     assert np.array_equal(state.cpu().numpy(), want["packed"])
     assert counts.tolist() == want["counts"].tolist()
     assert np.array_equal(rms.cpu().numpy().view(np.uint32), want["row_rms"].view(np.uint32))
+
+
+# (source, columns): every class that test_row_counts does not reach
+WIDE = [("f32", 1032), ("f32", 2312), ("bf16", 2056), ("bf16", 6664), ("splits", 2056),
+        ("splits", 6664), ("one split", 64), ("one split", 2056), ("one split", 6664)]
+
+
+@pytest.mark.parametrize("rows", [1, 5, 9, 17])
+@pytest.mark.parametrize("source,k", WIDE)
+def test_wide_rows(cuda, rows, source, k):
+    test_row_counts(cuda, rows, source, k)
+
+
+@pytest.mark.parametrize("rows,cut", [(16391, 8201), (2048, 2047), (768, 767)])
+@pytest.mark.parametrize("source,k", [("bf16", 64), ("bf16", 520), ("f32", 264), ("splits", 64),
+                                      ("splits", 1032), ("one split", 520), *WIDE])
+def test_rows_in_one_call_and_in_two(cuda, source, k, rows, cut):
+    from local_ai_training.ops import ratchet
+
+    gen = torch.Generator(cuda).manual_seed(k)
+    code = torch.randint(0, 7, (rows, k), generator=gen, device=cuda, dtype=torch.uint8)
+    pressure = torch.randint(0, 15, (rows, k), generator=gen, device=cuda, dtype=torch.uint8)
+    packed = code | (pressure << 4)
+    splits = {"splits": 3}.get(source, 1)
+    parts = torch.randn(splits, rows, k, generator=gen, device=cuda)
+
+    def run(first, last):
+        counts = torch.zeros(4, dtype=torch.int64, device=cuda)
+        rms = torch.empty(last - first, device=cuda)
+        state = packed[first:last].clone()
+        rule = (3, 8, 0.5, 1.5, 1e-8, None, 0.0, counts, rms, None, None, None)
+        if "split" in source:
+            ratchet().update_from_partials(state, parts[:, first:last].contiguous(), *rule, None)
+        else:
+            grad = parts[0, first:last]
+            ratchet().update_from_grad(state, grad.bfloat16() if source == "bf16" else grad, *rule)
+        return state, counts, rms
+
+    state, counts, rms = run(0, rows)
+    low, high = run(0, cut), run(cut, rows)
+    assert torch.equal(state, torch.cat([low[0], high[0]])) and not torch.equal(state, packed)
+    assert torch.equal(counts, low[1] + high[1])
+    assert torch.equal(rms.view(torch.int32), torch.cat([low[2], high[2]]).view(torch.int32))
