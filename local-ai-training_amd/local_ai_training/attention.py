@@ -66,12 +66,20 @@ def attention_supported(q: Tensor, k: Tensor, v: Tensor) -> bool:
 
 
 def _backward_fits(tensors: tuple[Tensor, ...]) -> bool:
-    """What ``rk_attention_backward`` takes: head size 128, and the limits of its 32-bit
-    offsets (one head's rows up to the padded length within 2^31 bytes of bf16, and all rows'
-    two float32 statistics)."""
+    """What ``rk_attention_backward`` takes (head size 128, and the limits of its 32-bit offsets:
+    one head's rows up to the padded length within 2^31 bytes of bf16, and all rows' two float32
+    statistics), where it is the faster one.
+
+    torch's kernel walks a head of up to 128 positions in one block; the HIP pair is two
+    launches of 128-row blocks. Device time in us, torch / HIP: 16 heads in all S 48 8.9 / 14.7,
+    S 128 14.7 / 23.3, S 160 36.9 / 24.7; 64 heads S 112 20.7 / 23.5, S 128 25.9 / 24.0; 128 heads
+    S 48 13.4 / 15.2, S 64 22.4 / 15.9; 256 heads S 16 9.0 / 11.6, S 32 18.9 / 12.9; 1024 heads
+    S 12 22.0 / 22.7, S 24 63.2 / 25.8. So up to 128 positions HIP takes 24 or more with at least
+    8192 positions over all heads."""
     b, h, s, d = tensors[0].shape
     padded = -(-s // 128) * 128
-    return (d == 128 and 8 * b * h * padded < 2**31
+    return (d == 128 and (s > 128 or s >= 24 and b * h * s >= 8192)
+            and 8 * b * h * padded < 2**31
             and ((padded + 64) * max(t.stride(2) for t in tensors) + d) * 2 < 2**31)
 
 
