@@ -61,7 +61,8 @@ __device__ __forceinline__ float half_sum(float v) {
 // probabilities are rounded to bf16 relative to the max after them, so U is part of the result's
 // rounding, which int8 rows downstream turn into differences of 1%: 64 at D = 64, 32 at D = 128.
 // With 64 at D = 128 too, B 8, H 16, S 1024 took 55-59 us against 59-61, B 2, H 8, S 2048 48
-// against 52.
+// against 52. R is 64, but 32 at D = 128 up to 32 positions: one step either way, in half the
+// LDS, so twice the blocks of a CU (8192 heads of 8 positions 35 us against 56).
 template <int D, int R, int U>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4)))
 void attn_fwd_kernel(AttnArgs a) {
@@ -269,6 +270,7 @@ extern "C" int rk_attention_forward(const uint16_t* q, int64_t sqb, int64_t sqh,
     a.BH = B * H - a.bh0 < per ? B * H - a.bh0 : per;
     const dim3 grid(static_cast<unsigned>(a.BH * nqb));
     if (D == 64) attn_fwd_kernel<64, 64, 64><<<grid, 256, 0, as_stream(stream)>>>(a);
+    else if (S <= 32) attn_fwd_kernel<128, 32, 32><<<grid, 256, 0, as_stream(stream)>>>(a);
     else attn_fwd_kernel<128, 64, 32><<<grid, 256, 0, as_stream(stream)>>>(a);
   }
   return launch_status("attention_forward");
