@@ -274,9 +274,11 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
     // Register-resident row (or row slice): one HBM read.
     const int c0 = slice * NC;  // this wavefront's first chunk
     float xr[NC][V];
-    if constexpr (VEC) {
+    if constexpr (VEC && NC > 1 && !(SRC == SRC_RMSNORM && DT == RK_F32)) {
       // every chunk's load in flight before the first is used; lanes past the row read its
-      // first vector (in bounds) and take zeros
+      // first vector (in bounds) and take zeros (us, one by one / all: 8192 x 2048 GELU bf16 18.8
+      // / 15.6, plain float32 19.5 / 18.2, RMSNorm bf16 14.6 / 14.0; a single chunk 16384 x 512
+      // bf16 10.2 / 10.5 and the float32 RMSNorm 5003 x 1040 7.5 / 7.9 are better off without)
       uint4 raw[NC];
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
@@ -292,7 +294,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(QuantArgs a) {
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         const int64_t e0 = (c0 + c) * SPAN + lane0;
-        if (c0 + c < nchunks) {
+        if (c0 + c < nchunks && (!VEC || e0 < a.K)) {
           load_chunk<DT, SRC, VEC>(a, row, e0, xr[c]);
         } else {
 #pragma unroll
