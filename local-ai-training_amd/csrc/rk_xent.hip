@@ -168,21 +168,28 @@ __global__ __launch_bounds__(1024) void xent_reduce_kernel(XentArgs a, float* lo
   const int tid = threadIdx.x;
   float sum = 0.0f;
   int n = 0;
-  // eight rows' loads in flight before their adds (the adds stay in row order)
-  for (int64_t r = tid; r < a.M; r += 8 * 1024) {
-    int64_t target[8];
-    float loss[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int64_t i = r + 1024 * j < a.M ? r + 1024 * j : r;
-      target[j] = a.targets[i];
-      loss[j] = a.stats[2 * a.M + i];
+  if (a.M <= 1024) {  // one row per thread
+    if (tid < a.M && a.targets[tid] != a.ignore) {
+      sum = sum + a.stats[2 * a.M + tid];
+      n = 1;
     }
+  } else {
+    // eight rows' loads in flight before their adds (the adds stay in row order)
+    for (int64_t r = tid; r < a.M; r += 8 * 1024) {
+      int64_t target[8];
+      float loss[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (r + 1024 * j < a.M && target[j] != a.ignore) {
-        sum = sum + loss[j];
-        ++n;
+      for (int j = 0; j < 8; ++j) {
+        const int64_t i = r + 1024 * j < a.M ? r + 1024 * j : r;
+        target[j] = a.targets[i];
+        loss[j] = a.stats[2 * a.M + i];
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (r + 1024 * j < a.M && target[j] != a.ignore) {
+          sum = sum + loss[j];
+          ++n;
+        }
       }
     }
   }
