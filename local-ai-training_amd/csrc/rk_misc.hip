@@ -244,9 +244,10 @@ extern "C" int rk_unpack(const uint8_t* packed, int64_t n, int max_code, int8_t*
   if (n < 0) return fail(RK_ERR_ARG, "negative size");
   if (n == 0) return RK_OK;
   if (!packed) return fail(RK_ERR_ARG, "null packed state");
-  // (a null code or pressure counts as aligned)
-  if (aligned16(packed) && aligned16(code) && aligned16(pressure) && max_code >= 0 &&
-      max_code <= 15) {
+  // (a null code or pressure counts as aligned; a byte per thread is no slower up to one byte for
+  // each thread the chip holds: 65536 weights 2.4 / 2.5 us, 1.1 M 3.6 / 2.7)
+  if (n >= (int64_t{1} << 17) && aligned16(packed) && aligned16(code) &&
+      aligned16(pressure) && max_code >= 0 && max_code <= 15) {
     unpack_vec_kernel<<<flat_grid(n, 16), 256, 0, as_stream(stream)>>>(packed, n, max_code, code,
                                                                        pressure);
   } else {

@@ -1,5 +1,5 @@
 """``unpack`` of the packed state at every alignment: 16-byte vectors where all three pointers
-allow them, with a tail of n % 16 bytes, and byte by byte otherwise. Exact."""
+allow them (from 2^17 bytes on), with a tail of n % 16 bytes, and byte by byte otherwise. Exact."""
 
 from __future__ import annotations
 
@@ -11,7 +11,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 15, 16, 17, 4095, 4096, 100_003])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4095, 4096, 100_003, 2**17 - 1, 2**17, 2**17 + 15])
 @pytest.mark.parametrize("offset", [0, 1, 16])
 def test_unpack_matches_the_nibbles(cuda, n, offset):
     from local_ai_training import _native as nat
