@@ -24,7 +24,6 @@ import math
 import torch
 import torch.nn.functional as F
 from torch import Tensor
-from torch.autograd.function import once_differentiable
 
 from .ops import ratchet
 
@@ -83,19 +82,6 @@ def _backward_fits(tensors: tuple[Tensor, ...]) -> bool:
             and ((padded + 64) * max(t.stride(2) for t in tensors) + d) * 2 < 2**31)
 
 
-def _attention_gradients(ctx, grad_out: Tensor) -> tuple[Tensor, Tensor, Tensor]:
-    q, k, v, out, lse = ctx.saved_tensors
-    if _backward_fits((q, k, v, out, grad_out)):
-        return ratchet().attention_backward(grad_out, q, k, v, out, lse, ctx.scale)
-    seed, offset = _philox_placeholders()
-    dq, dk, dv, _ = torch.ops.aten._scaled_dot_product_efficient_attention_backward(
-        grad_out, q, k, v, None, out, lse, seed, offset, 0.0, [True, True, True, False], True)
-    return dq, dk, dv
-
-
-_once_differentiable_gradients = once_differentiable(_attention_gradients)
-
-
 class CausalAttentionFn(torch.autograd.Function):
     """o = causal softmax(q k^T / sqrt(D)) v: HIP forward, HIP backward at head size 128."""
 
@@ -109,9 +95,15 @@ class CausalAttentionFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out: Tensor):
-        if torch.is_grad_enabled():  # create_graph: the gradients, but no second derivative
-            return _once_differentiable_gradients(ctx, grad_out)
-        return _attention_gradients(ctx, grad_out)
+        q, k, v, out, lse = ctx.saved_tensors
+        # create_graph: torch's operator, which knows that its results depend on q, k and v
+        # (and refuses their derivative), batched gradients included
+        if not torch.is_grad_enabled() and _backward_fits((q, k, v, out, grad_out)):
+            return ratchet().attention_backward(grad_out, q, k, v, out, lse, ctx.scale)
+        seed, offset = _philox_placeholders()
+        dq, dk, dv, _ = torch.ops.aten._scaled_dot_product_efficient_attention_backward(
+            grad_out, q, k, v, None, out, lse, seed, offset, 0.0, [True, True, True, False], True)
+        return dq, dk, dv
 
 
 def causal_attention(q: Tensor, k: Tensor, v: Tensor) -> Tensor:

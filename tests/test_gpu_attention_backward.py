@@ -119,3 +119,32 @@ def test_opcheck(cuda):
     q, k, v, g = inputs(cuda, 2, 2, 40, D)
     o, lse = ratchet().attention_forward(q, k, v, 0.125)
     torch.library.opcheck(ratchet().attention_backward, (g, q, k, v, o, lse, 0.125))
+
+
+@pytest.mark.parametrize("s,d", [(140, 128), (40, 128), (40, 64)])
+def test_a_second_derivative_is_refused_whatever_requires_grad(cuda, s, d):
+    """The gradients depend on q, k and v also where the output's gradient is a constant: a
+    penalty on them must raise, not leave its share out."""
+    leaves = [t.detach().requires_grad_() for t in inputs(cuda, 1, 2, s, d)[:3]]
+    out = causal_attention(*leaves)
+    first = torch.autograd.grad(out.float().sum(), leaves, create_graph=True)
+    check([a.detach() for a in first], (*(t.detach() for t in leaves), torch.ones_like(out)))
+    for a in first:
+        assert a.requires_grad
+        with pytest.raises(RuntimeError):
+            torch.autograd.grad(out.float().sum() + a.float().square().sum(), leaves,
+                                retain_graph=True)
+
+
+@pytest.mark.parametrize("create_graph", [False, True])
+@pytest.mark.parametrize("s,d", [(140, 128), (40, 128), (40, 64)])
+def test_batched_gradients(cuda, s, d, create_graph):
+    leaves = [t.detach().requires_grad_() for t in inputs(cuda, 2, 2, s, d)[:3]]
+    out = causal_attention(*leaves)
+    grads = torch.randn(3, *out.shape, device=cuda).bfloat16()
+    got = torch.autograd.grad(out, leaves, grads, retain_graph=True, create_graph=create_graph,
+                              is_grads_batched=True)
+    one = [torch.autograd.grad(out, leaves, g, retain_graph=True, create_graph=create_graph)
+           for g in grads]
+    for mine, single in zip(got, zip(*one)):
+        assert mine.requires_grad == create_graph and torch.equal(mine, torch.stack(single))
