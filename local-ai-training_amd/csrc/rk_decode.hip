@@ -97,7 +97,7 @@ __device__ __forceinline__ void dec_store_q(const float (&xr)[NC][4], int c0, in
       bool exact = false;
       float t[V];
 #pragma unroll
-      for (int i = 0; i < V; ++i) t[i] = round_fast<false>(xr[c][i], r, 0.0f, exact);
+      for (int i = 0; i < V; ++i) t[i] = round_fast(xr[c][i], r, exact);
       if (exact) {
 #pragma unroll
         for (int i = 0; i < V; ++i) t[i] = round_quotient<false>(xr[c][i], s, r, 0.0f);

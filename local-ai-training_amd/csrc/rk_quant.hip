@@ -179,7 +179,7 @@ __device__ __forceinline__ void quant_store_chunk(const QuantArgs& a, uint32_t c
   } else {
     bool exact = false;
 #pragma unroll
-    for (int i = 0; i < V; ++i) t[i] = round_fast<false>(y[i], r, 0.0f, exact);
+    for (int i = 0; i < V; ++i) t[i] = round_fast(y[i], r, exact);
     if (exact) {
       // a value of this lane's chunk lies within the margin of a rounding boundary (or is
       // not finite)

@@ -48,25 +48,16 @@ __device__ __forceinline__ float sr_fast(float y, float r, uint32_t w, float& wo
   return v;
 }
 
-// The fast path of round_quotient alone: the rounded value from ya = y * r, with `exact`
-// set (never cleared) where that value may differ from the one computed from y / s (the
-// same test as round_quotient's). Callers round a group of values this way and redo the
-// group with round_quotient only when some value set the flag, so the common case runs
-// without a branch per value.
-template <bool SR>
-__device__ __forceinline__ float round_fast(float y, float r, float u, bool& exact) {
+// The deterministic fast path of round_quotient alone: the rounded value from ya = y * r, with
+// `exact` set (never cleared) where that value may differ from the one computed from y / s (the
+// same test as round_quotient's). Callers round a group of values this way and redo the group
+// with round_quotient only when some value set the flag, so the common case runs without a
+// branch per value.
+__device__ __forceinline__ float round_fast(float y, float r, bool& exact) {
   const float ya = y * r;
-  if constexpr (SR) {
-    const float v = ya + u;
-    const float f = floorf(v);
-    const float d = v - f;
-    exact = exact || !(fabsf(ya) <= 128.0f) || d < kAmbiguity || d > 1.0f - kAmbiguity;
-    return f;
-  } else {
-    const float t = __builtin_rintf(ya);
-    exact = exact || !(fabsf(ya) <= 128.0f) || fabsf(ya - t) > 0.5f - kAmbiguity;
-    return t;
-  }
+  const float t = __builtin_rintf(ya);
+  exact = exact || !(fabsf(ya) <= 128.0f) || fabsf(ya - t) > 0.5f - kAmbiguity;
+  return t;
 }
 
 // Four int32 values in [-128, 127] as the bytes of one word (byte i from the i-th).
