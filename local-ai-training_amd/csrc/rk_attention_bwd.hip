@@ -1,6 +1,6 @@
 // Causal self-attention backward of the training step (gfx950), the backward of
-// rk_attention_forward at head size 128 (model.py:117-123): from bf16 q, k, v, o, do [B, H, S, D] and the
-// forward's log-sum-exp,
+// rk_attention_forward at head size 128 (model.py:117-123): from bf16 q, k, v, o, do [B, H, S, D]
+// and the forward's log-sum-exp,
 //   p_ij = exp(scale q_i . k_j - lse_i)   (j <= i, else 0),     delta_i = do_i . o_i,
 //   ds_ij = p_ij (do_i . v_j - delta_i),
 //   dq_i = scale sum_j ds_ij k_j,  dk_j = scale sum_i ds_ij q_i,  dv_j = sum_i p_ij do_i.
@@ -26,7 +26,8 @@
 // -delta, so neither needs a subtraction per element.
 //
 // Tiles are staged by LDS-DMA in two stages, one barrier per step (rk_attention.h). Heads run
-// fastest over the blocks, so that the blocks of one head share an XCD's L2.
+// fastest over the blocks: where their number is a multiple of 8, the blocks of one head share an
+// XCD's L2.
 //
 // B 8, H 16, S 1024: 73 + 92 us, 120 GFLOP at 730 TFLOP/s, against 293 us for torch's
 // memory-efficient backward (its kernel, the delta pass, and the float32 dq buffer cleared and
@@ -66,8 +67,8 @@ void attn_bwd_dq_kernel(AttnBwdArgs a) {
   const uint32_t lds0 = lds_address(smem);
   const int S = static_cast<int>(a.S);
   const int nqb = (S + kAttnRows - 1) / kAttnRows;
-  const int blk = static_cast<int>(blockIdx.x / a.BH);  // heads fastest: one head stays on an XCD
-  const int qb = nqb - 1 - blk;  // longest causal rows first
+  const int blk = static_cast<int>(blockIdx.x / a.BH);  // heads fastest
+  const int qb = nqb - 1 - blk;                         // longest causal rows first
   const int64_t bh = blockIdx.x - blk * a.BH, b = bh / a.H, hd = bh - b * a.H;
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -168,7 +169,7 @@ void attn_bwd_dkv_kernel(AttnBwdArgs a) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[VTILE + kAttnStages * STAGE];
   const uint32_t lds0 = lds_address(smem) + VTILE;
   const int S = static_cast<int>(a.S);
-  const int blk = static_cast<int>(blockIdx.x / a.BH);  // heads fastest: one head stays on an XCD
+  const int blk = static_cast<int>(blockIdx.x / a.BH);  // heads fastest
   const int64_t bh = blockIdx.x - blk * a.BH, b = bh / a.H, hd = bh - b * a.H;
   const int k0 = blk * kAttnRows;  // the first keys have the longest walk
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;

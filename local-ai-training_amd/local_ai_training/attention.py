@@ -4,13 +4,15 @@ The reference attends with ``F.scaled_dot_product_attention(q, k, v, is_causal=T
 (``model.py:117-123``). Here the forward is ``rk_attention_forward`` (flash form on the bf16
 MFMA, ``csrc/rk_attention.hip``), which writes the output and the per-query log-sum-exp in
 the form torch's memory-efficient attention forward does; the backward is
-``rk_attention_backward`` (``csrc/rk_attention_bwd.hip``) at head size 128 (165 us at B 8,
-H 16, S 1024 against 293 us for torch's memory-efficient backward, which adds its float32 dq by
-atomics in an order that varies). At head size 64 it stays torch's memory-efficient backward,
-called on the forward's two tensors: the HIP kernels were faster there too (70 against 131 us
-at B 32, H 8, S 512), but any other rounding of those gradients moves the loss of the 25M
-training step by up to 1e-3 within four steps (through the stochastic rounding and the update's
-thresholds), above the 5e-4 that step is held to (``perf/cases.py``).
+``rk_attention_backward`` (``csrc/rk_attention_bwd.hip``) at head size 128 where that is the
+faster one (``_backward_fits``): 165 us at B 8, H 16, S 1024 against 293 us for torch's
+memory-efficient backward, which adds its float32 dq by atomics in an order that varies from
+1024 positions on. Both are equally far from float64 (relative errors of dq, dk, dv 2.48e-3,
+2.46e-3, 2.30e-3 there, the same to three digits at 96 to 2048 positions and for scores of three
+times the size). Elsewhere, and at head size 64, it is torch's memory-efficient backward, called
+on the forward's two tensors. The same two HIP kernels at head size 64 took 70 us against 131 at
+B 32, H 8, S 512; they are not in use, for no lack of accuracy: they round differently, and the
+stochastic rounding and the update's thresholds downstream turn on last bits.
 
 Supported: bfloat16 GPU q, k, v [B, H, S, D] with D 64 or 128, unit feature stride,
 16-byte aligned storage and strides that are multiples of 8 elements, no attention mask,

@@ -221,8 +221,10 @@ def _attend(q: Tensor, k: Tensor, v: Tensor, **kwargs) -> Tensor:
     260 us against the flash kernel's 348 us at B 32, H 8, S 512, D 64, and 550 against
     885 us at B 8, H 16, S 1024, D 128, with the same forward output. Its backward at head
     size 128 accumulates dq in an order that varies from run to run (measured: dk, dv and
-    the output repeat bit for bit, dq does not; the flash kernel repeats at both shapes), so
-    under torch.use_deterministic_algorithms(True) the flash kernel comes first."""
+    the output repeat bit for bit, dq does not from 1024 positions on; the flash kernel repeats
+    at both shapes), so under torch.use_deterministic_algorithms(True) the flash kernel comes
+    first. Causal training attention otherwise runs the HIP kernels (attention.py), which
+    repeat; deterministic mode keeps the kernel it has had."""
     if q.is_cuda and q.dtype in (torch.bfloat16, torch.float16):
         deterministic = torch.are_deterministic_algorithms_enabled()
         if (hip_attention_forward and not deterministic and kwargs.get("is_causal")

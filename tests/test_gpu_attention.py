@@ -5,7 +5,8 @@ forward it replaces, ``F.scaled_dot_product_attention(q, k, v, is_causal=True)``
 Checked against the float64 softmax on the CPU (the mathematical values: o within one bf16
 rounding of the output plus the bf16 rounding of the probabilities, lse within float32
 rounding), against torch's own memory-efficient forward on the GPU, and through the backward
-(torch's memory-efficient backward fed our o and lse) against torch's whole attention.
+that each shape takes (the HIP one, or torch's memory-efficient backward fed our o and lse)
+against torch's whole attention.
 Shapes: the 25M (B 32, H 8, S 512, D 64) and 1B (B 8, H 16, S 1024, D 128) attention with the
 model's strided q/k/v views, and ragged sequence lengths.
 """
@@ -94,8 +95,9 @@ def test_matches_torch_forward_and_output_layout(cuda):
 
 @pytest.mark.parametrize("b,h,s,d", [(4, 8, 512, 64), (2, 16, 1024, 128), (2, 3, 129, 64)])
 def test_gradients_match_torch_attention(cuda, b, h, s, d):
-    """The HIP forward with torch's memory-efficient backward against torch's attention
-    (the efficient kernel's forward and backward), same inputs and output gradient."""
+    """The HIP forward with its backward (HIP at S 1024, D 128, torch's memory-efficient one at
+    D 64) against torch's attention (the efficient kernel's forward and backward), same inputs
+    and output gradient."""
     print(f"attention backward {b}x{h}x{s}x{d}", flush=True)
     q, k, v = qkv_views(b, h, s, d, cuda, seed=3 * s)
     go = torch.randn(b, h, s, d, generator=torch.Generator().manual_seed(4)).to(
